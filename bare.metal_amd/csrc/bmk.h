@@ -24,6 +24,8 @@ typedef struct {
     size_t      bytes[BMK_MAX_BUFFERS];    /* bytes available from the offset to the end */
     int         grid[3];                   /* Metal-style total threads */
     int         tg[3];                     /* Metal-style threadgroup size */
+    void*       scratch;                   /* the context's scratch memory, 256-byte aligned; its launches run in */
+    size_t      scratch_bytes;             /*   stream order, so each may use all of it (0: none could be allocated) */
 } bmk_launch_t;
 
 /* Returns 0 when the kernel was launched, -1 when the arguments were

@@ -9,7 +9,6 @@
  *       rmsnorm_forward_v2      reference src/kernels/forward.metal:1019-1060
  *       rope_forward            forward.metal:1260-1313
  *       kv_store                forward.metal:1317-1329
- *       attention_forward       forward.metal:1362-1465
  *       add_forward             forward.metal:1332-1340
  *       swiglu_forward          forward.metal:1179-1190
  *       rmsnorm_matmul_forward  forward.metal:1636-1689
@@ -130,81 +129,6 @@ __device__ __forceinline__ unsigned long long block_argmax_key(unsigned long lon
 }
 
 /* ================================================================== */
-/* Attention for one query head (one workgroup):
- *   out[d] = sum_t softmax_t(scale * q.k_t) v_t[d],  t < S.
- * Keys t < n_cached come from the cache rows kc/vc (stride KV floats); when
- * cur_k (LDS) is given, key t == n_cached == S-1 is cur_k/cur_v, used from
- * registers so that no pointer ever selects between LDS and global memory.
- * Online softmax over chunks of ATT_CH scores held in LDS.  HD divides 256. */
-__device__ void attn_head(const float* qs, const float* kc, const float* vc, int KV, int S, int n_cached,
-                          const float* cur_k, const float* cur_v, int HD, float scale, float* sc, float* red,
-                          float* sh, float* out) {
-    const int t = threadIdx.x;
-    const int G = NT / HD, g = t / HD, d = t - g * HD;
-    float s_cur = 0.0f, v_cur = 0.0f;
-    if (cur_k) {
-        float c0 = 0.f, c1 = 0.f;
-        for (int e = 0; e < HD; e += 2) {
-            c0 = fmaf(qs[e], cur_k[e], c0);
-            c1 = fmaf(qs[e + 1], cur_k[e + 1], c1);
-        }
-        s_cur = (c0 + c1) * scale;
-        v_cur = cur_v[d];
-    }
-    float m_run = -INFINITY, l_run = 0.0f, acc = 0.0f;
-    for (int base = 0; base < S; base += ATT_CH) {
-        const int n = min(ATT_CH, S - base);
-        float lmax = -INFINITY;
-        for (int i = t; i < n; i += NT) {
-            const int tt = base + i;
-            float s;
-            if (tt < n_cached) {
-                const float* kr = kc + (size_t)tt * KV;
-                float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
-                for (int e = 0; e < HD; e += 4) {
-                    float4 kv4;
-                    __builtin_memcpy(&kv4, __builtin_assume_aligned(kr + e, 4), 16);
-                    s0 = fmaf(qs[e + 0], kv4.x, s0);
-                    s1 = fmaf(qs[e + 1], kv4.y, s1);
-                    s2 = fmaf(qs[e + 2], kv4.z, s2);
-                    s3 = fmaf(qs[e + 3], kv4.w, s3);
-                }
-                s = ((s0 + s1) + (s2 + s3)) * scale;
-            } else {
-                s = s_cur;
-            }
-            sc[i] = s;
-            lmax = fmaxf(lmax, s);
-        }
-        const float cmax = block_max(lmax, sh);
-        float lsum = 0.0f;
-        for (int i = t; i < n; i += NT) {
-            const float p = expf(sc[i] - cmax);
-            sc[i] = p;
-            lsum += p;
-        }
-        const float csum = block_sum(lsum, sh); /* its barriers also publish sc[] */
-        const float m_new = fmaxf(m_run, cmax);
-        const float a_old = expf(m_run - m_new), a_new = expf(cmax - m_new);
-        l_run = l_run * a_old + csum * a_new;
-        float part = 0.0f;
-        const int n_c = min(n, n_cached - base); /* keys of this chunk that are in the cache */
-        for (int i = g; i < n_c; i += G) part = fmaf(sc[i], vc[(size_t)(base + i) * KV + d], part);
-        if (n_c < n && g == (n_c % G) && n_c >= 0) part = fmaf(sc[n_c], v_cur, part);
-        acc = acc * a_old + part * a_new;
-        m_run = m_new;
-        __syncthreads(); /* sc[] is rewritten by the next chunk */
-    }
-    red[g * HD + d] = acc;
-    __syncthreads();
-    if (t < HD) {
-        float s = 0.0f;
-        for (int k = 0; k < G; k++) s += red[k * HD + t];
-        out[t] = s / l_run;
-    }
-}
-
-/* ================================================================== */
 /* Reference-named kernels */
 
 __global__ __launch_bounds__(NT) void k_rmsnorm(const float* __restrict__ x, const float* __restrict__ w,
@@ -272,21 +196,6 @@ __global__ __launch_bounds__(NT) void k_kv_store(float* kvc, const float* k, con
     const size_t base = ((size_t)layer * 2 * MS + pos) * KV + i;
     kvc[base] = k[i];
     kvc[base + (size_t)MS * KV] = v[i];
-}
-
-__global__ __launch_bounds__(NT) void k_attention(const float* __restrict__ q, const float* __restrict__ kvc,
-                                                  float* __restrict__ out, int HD, int KV, int S, int kv_mul,
-                                                  int layer, int MS, float scale) {
-    __shared__ float qs[256];
-    __shared__ float sc[ATT_CH];
-    __shared__ float red[NT];
-    __shared__ float sh[4];
-    const int h = blockIdx.x, kh = h / kv_mul;
-    if (threadIdx.x < HD) qs[threadIdx.x] = q[h * HD + threadIdx.x];
-    __syncthreads();
-    const float* kc = kvc + (size_t)layer * 2 * MS * KV + kh * HD;
-    const float* vc = kc + (size_t)MS * KV;
-    attn_head(qs, kc, vc, KV, S, S, nullptr, nullptr, HD, scale, sc, red, sh, out + h * HD);
 }
 
 __global__ __launch_bounds__(NT) void k_add(const float* a, const float* b, float* out, int n) {
@@ -2049,28 +1958,6 @@ extern "C" int bmk_launch_kv_store(const bmk_launch_t* a) {
     BMK_NEED_BYTES(a, 2, (size_t)KV * 4, "v");
     hipLaunchKernelGGL(k_kv_store, dim3((KV + NT - 1) / NT), dim3(NT), 0, a->stream, (float*)a->dev[0],
                        (const float*)a->dev[1], (const float*)a->dev[2], layer, pos, MS, KV);
-    BMK_LAUNCH_CHECK();
-    return 0;
-}
-
-/* attention_forward {q [NH][HD], kv cache, out [NH][HD],
- *                    params int{NH, HD, NKV, KV, S, kv_mul, layer, MS}, scale float} */
-extern "C" int bmk_launch_attention(const bmk_launch_t* a) {
-    BMK_NEED_BYTES(a, 3, 32, "params");
-    BMK_NEED_BYTES(a, 4, 4, "scale");
-    const int NH = bmk_pi(a, 3, 0), HD = bmk_pi(a, 3, 1), KV = bmk_pi(a, 3, 3), S = bmk_pi(a, 3, 4);
-    const int kv_mul = bmk_pi(a, 3, 5), layer = bmk_pi(a, 3, 6), MS = bmk_pi(a, 3, 7);
-    const float scale = bmk_pf(a, 4, 0);
-    BMK_REQUIRE(NH > 0 && HD > 0 && HD <= 256 && 256 % HD == 0 && HD % 4 == 0 && kv_mul > 0 && layer >= 0 && MS > 0 &&
-                    S >= 1 && S <= MS && ((NH - 1) / kv_mul + 1) * HD <= KV,
-                "attention: bad params NH=%d HD=%d KV=%d S=%d kv_mul=%d layer=%d MS=%d", NH, HD, KV, S, kv_mul, layer,
-                MS);
-    BMK_NEED_BYTES(a, 0, (size_t)NH * HD * 4, "q");
-    BMK_NEED_BYTES(a, 1, ((size_t)layer * 2 + 2) * MS * KV * 4, "kv cache");
-    BMK_NEED_BYTES(a, 2, (size_t)NH * HD * 4, "out");
-    BMK_REQUIRE(((uintptr_t)a->dev[1] & 15) == 0 && KV % 4 == 0, "attention: kv cache rows must be 16-byte aligned");
-    hipLaunchKernelGGL(k_attention, dim3(NH), dim3(NT), 0, a->stream, (const float*)a->dev[0], (const float*)a->dev[1],
-                       (float*)a->dev[2], HD, KV, S, kv_mul, layer, MS, scale);
     BMK_LAUNCH_CHECK();
     return 0;
 }

@@ -62,6 +62,8 @@ static bool hip_ok(hipError_t e, const char* what, const char* file, int line) {
     return false;
 }
 
+#define BMK_SCRATCH_BYTES ((size_t)8 << 20)
+
 static inline hipStream_t ctx_stream(backend_ctx_t* ctx) { return (hipStream_t)ctx->queue; }
 
 static void ctx_sync(backend_ctx_t* ctx) {
@@ -91,6 +93,15 @@ extern "C" backend_ctx_t* backend_create(void) {
         free(ctx);
         return NULL;
     }
+    /* a context's launches run in the order of its one stream, so they share one scratch memory; without
+     * it the kernels that would split their work run unsplit */
+    if (hipMalloc(&ctx->scratch, BMK_SCRATCH_BYTES) == hipSuccess &&
+        hipMemsetAsync(ctx->scratch, 0, BMK_SCRATCH_BYTES, s) == hipSuccess) {
+        ctx->scratch_bytes = BMK_SCRATCH_BYTES;
+    } else {
+        (void)hipGetLastError();
+        BMK_WARN("backend_create: no scratch memory, kernels run unsplit");
+    }
     ctx->device = (void*)(intptr_t)dev;
     ctx->queue = (void*)s;
     ctx->library = (void*)bmk_table;
@@ -114,6 +125,7 @@ extern "C" void backend_destroy(backend_ctx_t* ctx) {
         ctx_sync(ctx);
         HIP_OK(hipStreamDestroy(ctx_stream(ctx)), "hipStreamDestroy");
     }
+    if (ctx->scratch) HIP_OK(hipFree(ctx->scratch), "hipFree");
     for (int i = 0; i < ctx->n_event_pool; i++)
         HIP_OK(hipEventDestroy((hipEvent_t)ctx->event_pool[i]), "hipEventDestroy");
     free(ctx);
@@ -325,6 +337,8 @@ extern "C" int backend_encode_dispatch(backend_encoder_t* enc, backend_kernel_t*
     memset(&a, 0, sizeof a);
     a.stream = ctx_stream(ctx);
     a.n = num_buffers;
+    a.scratch = ctx->scratch;
+    a.scratch_bytes = ctx->scratch_bytes;
     a.grid[0] = grid_x; a.grid[1] = grid_y; a.grid[2] = grid_z;
     a.tg[0] = tg_x; a.tg[1] = tg_y; a.tg[2] = tg_z;
     for (int i = 0; i < num_buffers; i++) {

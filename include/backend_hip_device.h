@@ -46,6 +46,11 @@ struct backend_ctx_s {
     /* Recycled hipEvent_t pairs for encoders. */
     void*  event_pool[32];
     int    n_event_pool;
+
+    /* Device memory for kernels that split their work and merge it (zeroed
+     * at creation; NULL and 0 when it could not be allocated). */
+    void*  scratch;
+    size_t scratch_bytes;
 };
 
 struct backend_buffer_s {

@@ -153,6 +153,49 @@ def test_attention_forward(be, NH, NKV, HD, S, MS):
     assert nw(out.read(np.float32), want) <= TOL
 
 
+@pytest.mark.parametrize("NH,kv_mul,HD", [(15, 3, 64), (14, 5, 64), (3, 1, 128), (9, 8, 32), (2, 2, 256), (5, 4, 4),
+                                          (3, 7, 16)])
+@pytest.mark.parametrize("S", [1, 63, 64, 65, 129, 193, 1000, 4097])
+def test_attention_forward_splits(be, NH, kv_mul, HD, S):
+    """Key counts around the split's tiles (one split up to two tiles, then one per tile, then several tiles per
+    split), head groups that kv_mul and NH do not fill, each launched twice with the cache's other rows NaN (past S)
+    and the output buffer's old contents NaN; fp32 sums against 64 bits as above."""
+    rng = np.random.default_rng(S * HD + NH)
+    NKV = (NH - 1) // kv_mul + 1
+    KV, MS = NKV * HD, S + 3
+    q = rng.standard_normal(NH * HD).astype(np.float32)
+    cache = (rng.standard_normal(2 * MS * KV) * 0.5).astype(np.float32)
+    dirty = cache.reshape(2, MS, KV).copy()
+    dirty[:, S:] = np.nan
+    scale = np.float32(1.0 / np.sqrt(HD))
+    want = attn_ref(q, cache, NH, HD, KV, S, kv_mul, 0, MS, scale)
+    out = be.upload(np.full(NH * HD, np.nan, np.float32))
+    bufs = [be.upload(q), be.upload(dirty), out, be.params(NH, HD, NKV, KV, S, kv_mul, 0, MS), be.upload(f32(scale))]
+    for _ in range(2):
+        assert be.dispatch("attention_forward", bufs, (NH * HD,), (HD,)) == 0
+    assert nw(out.read(np.float32), want) <= TOL
+
+
+def test_attention_forward_masked_and_nonfinite(be):
+    """Scores of -inf drop their keys (here all but one key of one split), scores that are all -inf, +inf or NaN give
+    NaN, as the unsplit softmax has them."""
+    HD, S, inf, nan = 64, 300, np.inf, np.nan
+    rng = np.random.default_rng(7)
+    v = rng.standard_normal((S, HD)).astype(np.float32)
+    q = np.zeros(HD, np.float32)
+    q[0] = 1.0
+    for scores, key in (([-inf] * 200 + [2.0] + [-inf] * 99, 200), ([-inf] * S, None), ([0.0] * 150 + [inf] + [0.0] * 149, None),
+                        ([0.0] * 299 + [nan], None), ([-inf] * 10 + [nan] + [-inf] * 289, None)):
+        cache = np.zeros((2, S, HD), np.float32)
+        cache[0, :, 0], cache[1] = scores, v
+        out = be.alloc(HD * 4)
+        assert be.dispatch("attention_forward", [be.upload(q), be.upload(cache), out,
+                                                 be.params(1, HD, 1, HD, S, 1, 0, S), be.upload(f32(1.0))],
+                           (HD,), (HD,)) == 0
+        got = out.read(np.float32)
+        assert np.array_equal(got, v[key]) if key is not None else np.isnan(got).all()
+
+
 def test_attention_single_key_is_v(be):
     NH, NKV, HD, MS = 9, 3, 64, 4
     KV = NKV * HD
