@@ -30,6 +30,7 @@
 #include "decode_state.h"
 #include "q8_common.h"
 #include "q8_gemm.h"
+#include "rows_gemm.h"
 
 #include <math.h>
 #include <string.h>
@@ -2167,11 +2168,13 @@ __global__ __launch_bounds__(NT) void k_matmul_rows_any(const float* __restrict_
  * matmul_forward_bf16_tiled / _tiled64 / _simd, 327-442
  * matmul_forward_fp16_vec / _fp16 / _fp16_tiled).  The reference's
  * prefill takes them for the LM head of its last position (graph.c:373-380,
- * selected by scheduler.c:1118-1145 and registry.c:60-67).  Served by the
- * LM-head kernel with the RMSNorm off where it tiles C (a multiple of 16 up
- * to 4096 for fp32 rows, of 32 up to 8192 for bf16): each workgroup loads
- * its weight rows once and applies them to all BT input rows.  Any other C
- * takes k_matmul_rows_any.  The grid the caller passes is not used. */
+ * selected by scheduler.c:1118-1145 and registry.c:60-67).  Several rows go
+ * to the fp32-MFMA matmul (rows_gemm.hip) where rows_gemm_ok.  The rest is
+ * served by the LM-head kernel with the RMSNorm off where it tiles C (a
+ * multiple of 16 up to 4096 for fp32 rows, of 32 up to 8192 for bf16): each
+ * workgroup loads its weight rows once and applies them to all BT input
+ * rows.  Any other C takes k_matmul_rows_any.  The grid the caller passes is
+ * not used. */
 static int launch_matmul_rows(const bmk_launch_t* a, int wf) {
     const char* name = wf == HW_F32 ? "matmul_forward (fp32)" : wf == HW_BF16 ? "matmul_forward_bf16" : "matmul_forward_fp16";
     const size_t esz = wf == HW_F32 ? 4 : 2;
@@ -2183,6 +2186,9 @@ static int launch_matmul_rows(const bmk_launch_t* a, int wf) {
     BMK_NEED_BYTES(a, 1, (size_t)OC * C * esz, "weight");
     if (hb) BMK_NEED_BYTES(a, 2, (size_t)OC * 4, "bias");
     BMK_NEED_BYTES(a, 3, (size_t)BT * OC * 4, "out");
+    if (rows_gemm_ok(BT, C, OC) && (((uintptr_t)a->dev[0] | (uintptr_t)a->dev[1]) & 3) == 0)
+        return rows_gemm_launch((const float*)a->dev[0], (const void*)a->dev[1], wf, hb ? (const float*)a->dev[2] : nullptr,
+                                (float*)a->dev[3], BT, C, OC, a->stream);
     if (!head_shape_ok(C, wf)) {
         BMK_REQUIRE(((uintptr_t)a->dev[0] & 3) == 0 && ((uintptr_t)a->dev[1] & (esz - 1)) == 0,
                     "%s: misaligned operand", name);

@@ -421,6 +421,44 @@ def test_plain_matmul_forward_rejects(be):
                        (32,), (32,)) == -1
 
 
+@pytest.mark.parametrize("BT,C,OC", [(2, 32, 1), (2, 1056, 20), (3, 576, 33), (31, 96, 64), (33, 160, 31), (64, 960, 320), (65, 8224, 40),
+                                     (200, 128, 2049), (512, 64, 2048)])
+@pytest.mark.parametrize("bias,off", [(0, 0), (1, 4)])
+@pytest.mark.parametrize("name", ["matmul_forward_fp32_tiled", "matmul_forward_bf16_simd", "matmul_forward_fp16_tiled"])
+def test_matmul_forward_rows(be, name, BT, C, OC, bias, off):
+    """Several rows over unquantized weights: both tile shapes (200 x 2049 and 512 x 2048 take the 64-row one), rows,
+    outputs and K steps that do not fill them, K shorter than a step, operands at 4-byte offsets; fp32 products and
+    sums against 64 bits over the same weights, and nothing written past the output."""
+    rng = np.random.default_rng(BT * C + OC)
+    x = rng.standard_normal((BT, C)).astype(np.float32)
+    w = (rng.standard_normal(OC * C) * 0.02).astype(np.float32)
+    wv, wb = (w, w) if "fp32" in name else _h16(w, name)
+    b = rng.standard_normal(OC).astype(np.float32)
+    out = be.upload(np.full(BT * OC + 64, 7.0, np.float32))
+    pad = np.zeros(off // 4, np.float32)
+    bx = be.upload(np.concatenate([pad, x.ravel()]))
+    bw = be.upload(np.concatenate([pad.view(np.uint8), wb.view(np.uint8)]))
+    assert be.dispatch(name, [bx, bw, be.upload(b), out, be.params(BT, C, OC, bias)], (OC, BT), (32,),
+                       offsets=[off, off, 0, 0, 0]) == 0
+    got = out.read(np.float32)
+    want = x.astype(np.float64) @ wv.reshape(OC, C).astype(np.float64).T + bias * b
+    assert nw(got[:BT * OC], want.ravel()) <= TOL
+    assert (got[BT * OC:] == 7.0).all()
+
+
+def test_matmul_forward_rows_nonfinite(be):
+    """An infinite or NaN operand reaches its own row and column only, as in the plain sum."""
+    BT, C, OC = 40, 256, 70
+    x, w = np.ones((BT, C), np.float32), np.ones((OC, C), np.float32)
+    x[3, 5], x[33, 200], w[69, 7] = np.inf, np.nan, -np.inf
+    out = be.alloc(BT * OC * 4)
+    assert be.dispatch("matmul_forward_fp32_tiled", [be.upload(x), be.upload(w), out, out, be.params(BT, C, OC, 0)],
+                       (OC, BT), (32,)) == 0
+    with np.errstate(invalid="ignore"):
+        want = (x.astype(np.float64)[:, None, :] * w.astype(np.float64)[None, :, :]).sum(axis=2)
+    np.testing.assert_array_equal(out.read(np.float32).reshape(BT, OC), want.astype(np.float32))
+
+
 def test_argmax_first_index(be):
     v = np.zeros(49152, np.float32)
     v[[10, 40000, 7]] = 2.5
