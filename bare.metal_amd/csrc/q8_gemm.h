@@ -52,6 +52,9 @@ int gm_tiles_frag(int M, int N);
 int gm_cast_bf16(const float* src, unsigned short* dst, long n, hipStream_t s);
 /* src fp32 [M][lda] -> dst bf16 [M][K] in MFMA fragment order (frag_index), padding zeroed */
 int gm_cast_bf16_frag(const float* src, unsigned short* dst, int M, int K, int lda, hipStream_t s);
+/* one GEMM C[M][N] = A[M][K] x W^T, fp32 A and C, qf as bmk::QF_* (q8_gemm_one.hip): 1 launched, 0 not a
+ * shape of its tiles (the 128 x 128 kernel's), -1 failed */
+int gm_launch_one(const float* A, const unsigned char* W, float* C, int M, int N, int K, int qf, hipStream_t s);
 int gm_launch_group(GmGroup* g, hipStream_t s);
 int gm_launch_group_qf(GmGroup* g, int qf, hipStream_t s);
 int gm_launch_multi_qf(const void* A, int a_bf16, int qf, const unsigned char* W, float* C, const void* plan,

@@ -583,47 +583,35 @@ extern "C" int gm_tiles_for(int M, int N) { return ((M + BM - 1) / BM) * ((N + B
 extern "C" int gm_tiles_frag(int M, int N) { return ((M + GM_FBM - 1) / GM_FBM) * ((N + GM_FBN - 1) / GM_FBN); }
 
 /* The tile loaders address a problem with 32-bit offsets. */
-static bool gm_offsets_fit(int M, int N, int K, int lda) {
-    return (unsigned long long)M * (unsigned long long)lda < 0x80000000ull &&
-           (unsigned long long)N * (unsigned long long)(K / 32) * 36ull < 0x80000000ull;
-}
-
-static bool gm_offsets_fit_q(int M, int N, int K, int lda, unsigned bytes) {
+static bool gm_offsets_fit(int M, int N, int K, int lda, unsigned bytes) {
     return (unsigned long long)M * (unsigned long long)lda < 0x80000000ull &&
            (unsigned long long)N * (unsigned long long)(K / 32) * bytes < 0x80000000ull;
 }
 
-/* The group launch over Q4_0 weights (qf 1) or Q8_0 (qf 0). */
+/* Problems by value (matmul_forward_q8 / _q4), over Q8_0 (qf 0) or Q4_0 (qf
+ * 1) weights; a single dense one with few tiles goes to the kernel made for it. */
 extern "C" int gm_launch_group_qf(GmGroup* g, int qf, hipStream_t s) {
-    if (qf == 0) return gm_launch_group(g, s);
     long total = 0;
-    for (int i = 0; i < g->nprob; i++)
-        BMK_REQUIRE(gm_offsets_fit_q(g->p[i].M, g->p[i].N, g->p[i].K, g->p[i].lda, 20u),
-                    "q4 gemm: problem %d too large for 32-bit tile offsets", i);
     for (int i = 0; i < g->nprob; i++) {
-        g->p[i].tiles = gm_tiles_for(g->p[i].M, g->p[i].N);
-        total += g->p[i].tiles;
+        GmProb& p = g->p[i];
+        BMK_REQUIRE(gm_offsets_fit(p.M, p.N, p.K, p.lda, qf ? 20u : 36u),
+                    "q%d gemm: problem %d too large for 32-bit tile offsets", qf ? 4 : 8, i);
+        p.tiles = gm_tiles_for(p.M, p.N);
+        total += p.tiles;
     }
     if (total <= 0) return 0;
-    hipLaunchKernelGGL(k_q4_gemm, dim3((unsigned)total), dim3(NTH), 0, s, *g);
+    const GmProb& p = g->p[0];
+    if (g->nprob == 1 && p.lda == p.K && p.ldc == p.N) {
+        const int rc = gm_launch_one(p.A, p.W, p.C, p.M, p.N, p.K, qf, s);
+        if (rc != 0) return rc > 0 ? 0 : -1;
+    }
+    if (qf) hipLaunchKernelGGL(k_q4_gemm, dim3((unsigned)total), dim3(NTH), 0, s, *g);
+    else hipLaunchKernelGGL(k_q8_gemm, dim3((unsigned)total), dim3(NTH), 0, s, *g);
     BMK_LAUNCH_CHECK();
     return 0;
 }
 
-extern "C" int gm_launch_group(GmGroup* g, hipStream_t s) {
-    long total = 0;
-    for (int i = 0; i < g->nprob; i++)
-        BMK_REQUIRE(gm_offsets_fit(g->p[i].M, g->p[i].N, g->p[i].K, g->p[i].lda),
-                    "q8 gemm: problem %d too large for 32-bit tile offsets", i);
-    for (int i = 0; i < g->nprob; i++) {
-        g->p[i].tiles = gm_tiles_for(g->p[i].M, g->p[i].N);
-        total += g->p[i].tiles;
-    }
-    if (total <= 0) return 0;
-    hipLaunchKernelGGL(k_q8_gemm, dim3((unsigned)total), dim3(NTH), 0, s, *g);
-    BMK_LAUNCH_CHECK();
-    return 0;
-}
+extern "C" int gm_launch_group(GmGroup* g, hipStream_t s) { return gm_launch_group_qf(g, 0, s); }
 
 /* matmul_forward_q8_multi: many independent prefill GEMMs in one launch.
  * buffers {0 params int {nprob, n_tiles[, a_bf16]} (by value; a_bf16 = 1: the
@@ -662,7 +650,7 @@ static int launch_gemm_multi(const bmk_launch_t* a) {
                     "q8 gemm multi: problem %d tiles %d@%d, expected %d@%ld", i, d.tiles, d.tile0, want_tiles,
                     next_tile);
         BMK_REQUIRE((d.w_off & 3) == 0, "q8 gemm multi: problem %d weight offset not 4-byte aligned", i);
-        BMK_REQUIRE(gm_offsets_fit_q(d.M, d.N, d.K, d.lda, BYTES),
+        BMK_REQUIRE(gm_offsets_fit(d.M, d.N, d.K, d.lda, BYTES),
                     "q8 gemm multi: problem %d too large for 32-bit tile offsets", i);
         BMK_REQUIRE((!a_bf16 || (d.a_off % 8 == 0 && d.lda % 8 == 0)),
                     "q8 gemm multi: problem %d bf16 rows must start 16-byte aligned", i);

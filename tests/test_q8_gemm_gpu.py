@@ -40,6 +40,44 @@ def test_gemm_vs_oracle(be, M, K, N):
     assert normwise(c, rx) <= 1e-2, normwise(c, rx)
 
 
+@pytest.mark.parametrize("M,K,N", [
+    (17, 32, 33), (33, 256, 95), (64, 800, 1000),          # 32 x 32 tiles: K below, at and past a 256-wide step
+    (100, 160, 2100), (100, 128, 2100), (97, 672, 2100),   # 32 x 64, steps of 128
+    (200, 416, 3100),                                      # 64 x 64
+    (300, 96, 4000), (300, 64, 4000),                      # 64 x 128, steps of 64
+    (600, 96, 4000),                                       # the 128 x 128 kernel
+])
+@pytest.mark.parametrize("qf", ["q8", "q4"])
+def test_gemm_tile_shapes(be, qf, M, K, N):
+    """Every tile shape matmul_forward_q8 / _q4 choose among, tiles that M and N do not fill, every kind of last K
+    step, against the bf16-operand product in 64 bits (fp32 summation order only: 1e-4), with the output's
+    neighbours and the weights of a following matrix (NaN scales) untouched and unread."""
+    rng = np.random.default_rng(M + K + N)
+    nb = K // 32
+    blk = np.zeros((N * nb + 8, 36 if qf == "q8" else 20), np.uint8)
+    blk[:, :4] = np.full(len(blk), np.nan, np.float32).view(np.uint8).reshape(-1, 4)
+    sc = rng.uniform(1e-4, 2e-3, N * nb).astype(np.float32)
+    blk[:N * nb, :4] = sc.view(np.uint8).reshape(-1, 4)
+    top = 127 if qf == "q8" else 7
+    code = rng.integers(-top, top + 1, (N * nb, 32)).astype(np.int8)
+    if qf == "q8":
+        blk[:N * nb, 4:] = code.view(np.uint8)
+    else:
+        nib = code.view(np.uint8) & 15
+        blk[:N * nb, 4:] = nib[:, 0::2] | (nib[:, 1::2] << 4)
+    a = rng.standard_normal((M, K)).astype(np.float32)
+    guard = np.full(M * N + 256, 3.0, np.float32)
+    bc = be.upload(guard)
+    ba = be.upload(np.concatenate([a.ravel(), np.full(K, np.nan, np.float32)]))
+    assert be.dispatch("matmul_forward_" + qf, [ba, be.upload(blk), be.alloc(4), bc, be.params(M, K, N, 0)],
+                       ((N + 31) & ~31, M), (32,)) == 0
+    c = bc.read(np.float32)
+    w = po.bf16_rne((code.astype(np.float32) * sc[:, None]).ravel()).reshape(N, K)
+    r = po.bf16_rne(a.ravel()).reshape(M, K).astype(np.float64) @ w.astype(np.float64).T
+    assert normwise(c[:M * N], r.ravel()) <= 1e-4
+    assert (c[M * N:] == 3.0).all()
+
+
 def test_gemm_integer_exact(be):
     rng = np.random.default_rng(2)
     M, K, N = 64, 128, 80
