@@ -72,6 +72,45 @@ static void ctx_sync(backend_ctx_t* ctx) {
 }
 
 /* ------------------------------------------------------------------ */
+/* events */
+
+/* A recycled event, counted: an encoder's stop event may be the next
+ * encoder's start event, and the context keeps the last one. */
+typedef struct {
+    hipEvent_t ev;
+    int refs;
+} bmk_event_t;
+
+static bmk_event_t* event_get(backend_ctx_t* ctx) {
+    if (ctx->n_event_pool > 0) {
+        bmk_event_t* e = (bmk_event_t*)ctx->event_pool[--ctx->n_event_pool];
+        e->refs = 1;
+        return e;
+    }
+    bmk_event_t* e = (bmk_event_t*)calloc(1, sizeof(bmk_event_t));
+    if (!e) return nullptr;
+    if (!HIP_OK(hipEventCreate(&e->ev), "hipEventCreate")) {
+        free(e);
+        return nullptr;
+    }
+    e->refs = 1;
+    return e;
+}
+
+static void event_destroy(bmk_event_t* e) {
+    HIP_OK(hipEventDestroy(e->ev), "hipEventDestroy");
+    free(e);
+}
+
+static void event_put(backend_ctx_t* ctx, bmk_event_t* e) {
+    if (!e || --e->refs > 0) return;
+    if (ctx->n_event_pool < (int)(sizeof ctx->event_pool / sizeof ctx->event_pool[0]))
+        ctx->event_pool[ctx->n_event_pool++] = (void*)e;
+    else
+        event_destroy(e);
+}
+
+/* ------------------------------------------------------------------ */
 /* context */
 
 extern "C" backend_ctx_t* backend_create(void) {
@@ -126,8 +165,8 @@ extern "C" void backend_destroy(backend_ctx_t* ctx) {
         HIP_OK(hipStreamDestroy(ctx_stream(ctx)), "hipStreamDestroy");
     }
     if (ctx->scratch) HIP_OK(hipFree(ctx->scratch), "hipFree");
-    for (int i = 0; i < ctx->n_event_pool; i++)
-        HIP_OK(hipEventDestroy((hipEvent_t)ctx->event_pool[i]), "hipEventDestroy");
+    event_put(ctx, (bmk_event_t*)ctx->last_stop);
+    for (int i = 0; i < ctx->n_event_pool; i++) event_destroy((bmk_event_t*)ctx->event_pool[i]);
     free(ctx);
 }
 
@@ -285,19 +324,35 @@ extern "C" void backend_kernel_destroy(backend_kernel_t* kernel) { free(kernel);
 /* ------------------------------------------------------------------ */
 /* encoders */
 
-static hipEvent_t event_get(backend_ctx_t* ctx) {
-    if (ctx->n_event_pool > 0) return (hipEvent_t)ctx->event_pool[--ctx->n_event_pool];
-    hipEvent_t e = nullptr;
-    if (!HIP_OK(hipEventCreate(&e), "hipEventCreate")) return nullptr;
+/* The event an encoder begins at.  Where nothing went onto the stream since
+ * the last encoder's stop event and the GPU has not reached that yet, an
+ * event recorded now would take its time stamp right behind it: the encoder
+ * starts at that event itself, one barrier packet less between the two
+ * encoders' kernels.  Encoders of one kernel kept in flight:
+ * 14.9 -> 10.9 us a pass for a 7.5 us kernel, 46.5 -> 42.7 for a 40 us one, 22.9 ->
+ * 18.0 for a 15.6 us one; an encoder on an idle stream is as before.  (Events
+ * that release to no more than the device save another 1.5 us there and cost
+ * 2.5 us where the host then waits for the whole device.) */
+static bmk_event_t* event_start(backend_ctx_t* ctx) {
+    bmk_event_t* last = (bmk_event_t*)ctx->last_stop;
+    if (last && ctx->last_stop_epoch == ctx->submit_epoch) {
+        /* the query is no part of a graph that this thread may be capturing on another stream */
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        const hipError_t q = hipEventQuery(last->ev);
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (q == hipErrorNotReady) {
+            last->refs++;
+            return last;
+        }
+        if (q != hipSuccess) (void)hipGetLastError();
+    }
+    bmk_event_t* e = event_get(ctx);
+    if (e && !HIP_OK(hipEventRecord(e->ev, ctx_stream(ctx)), "hipEventRecord")) {
+        event_put(ctx, e);
+        return nullptr;
+    }
     return e;
-}
-
-static void event_put(backend_ctx_t* ctx, hipEvent_t e) {
-    if (!e) return;
-    if (ctx->n_event_pool < (int)(sizeof ctx->event_pool / sizeof ctx->event_pool[0]))
-        ctx->event_pool[ctx->n_event_pool++] = (void*)e;
-    else
-        HIP_OK(hipEventDestroy(e), "hipEventDestroy");
 }
 
 extern "C" backend_encoder_t* backend_encode_begin(backend_ctx_t* ctx) {
@@ -305,7 +360,7 @@ extern "C" backend_encoder_t* backend_encode_begin(backend_ctx_t* ctx) {
     backend_encoder_t* e = (backend_encoder_t*)calloc(1, sizeof(backend_encoder_t));
     if (!e) return NULL;
     e->ctx = ctx;
-    hipEvent_t a = event_get(ctx), b = event_get(ctx);
+    bmk_event_t *a = event_start(ctx), *b = event_get(ctx);
     if (!a || !b) {
         event_put(ctx, a);
         event_put(ctx, b);
@@ -314,7 +369,6 @@ extern "C" backend_encoder_t* backend_encode_begin(backend_ctx_t* ctx) {
     }
     e->ev_start = (void*)a;
     e->ev_stop = (void*)b;
-    HIP_OK(hipEventRecord(a, ctx_stream(ctx)), "hipEventRecord");
     return e;
 }
 
@@ -378,8 +432,17 @@ extern "C" int backend_encode_dispatch(backend_encoder_t* enc, backend_kernel_t*
 
 extern "C" void backend_encode_commit(backend_encoder_t* enc) {
     if (!enc || enc->committed) return;
-    HIP_OK(hipEventRecord((hipEvent_t)enc->ev_stop, ctx_stream(enc->ctx)), "hipEventRecord");
-    enc->commit_epoch = enc->ctx->submit_epoch;
+    backend_ctx_t* ctx = enc->ctx;
+    bmk_event_t* stop = (bmk_event_t*)enc->ev_stop;
+    const bool recorded = HIP_OK(hipEventRecord(stop->ev, ctx_stream(ctx)), "hipEventRecord");
+    event_put(ctx, (bmk_event_t*)ctx->last_stop);
+    ctx->last_stop = NULL;
+    if (recorded) {
+        stop->refs++;
+        ctx->last_stop = (void*)stop;
+        ctx->last_stop_epoch = ctx->submit_epoch;
+    }
+    enc->commit_epoch = ctx->submit_epoch;
     enc->committed = 1;
 }
 
@@ -388,10 +451,10 @@ extern "C" double backend_encode_wait_timed(backend_encoder_t* enc) {
     backend_ctx_t* ctx = enc->ctx;
     if (!enc->committed) backend_encode_commit(enc);
     float ms = 0.0f;
-    hipEvent_t a = (hipEvent_t)enc->ev_start, b = (hipEvent_t)enc->ev_stop;
-    if (HIP_OK(hipEventSynchronize(b), "hipEventSynchronize")) {
+    bmk_event_t *a = (bmk_event_t*)enc->ev_start, *b = (bmk_event_t*)enc->ev_stop;
+    if (HIP_OK(hipEventSynchronize(b->ev), "hipEventSynchronize")) {
         if (enc->commit_epoch > ctx->done_epoch) ctx->done_epoch = enc->commit_epoch;
-        if (hipEventElapsedTime(&ms, a, b) != hipSuccess) {
+        if (hipEventElapsedTime(&ms, a->ev, b->ev) != hipSuccess) {
             (void)hipGetLastError();
             ms = 0.0f;
         }

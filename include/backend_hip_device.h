@@ -43,9 +43,12 @@ struct backend_ctx_s {
     uint64_t submit_epoch;
     uint64_t done_epoch;
 
-    /* Recycled hipEvent_t pairs for encoders. */
+    /* Recycled events of encoders, and the last committed encoder's stop
+     * event with the submit epoch it was recorded at. */
     void*  event_pool[32];
     int    n_event_pool;
+    void*  last_stop;
+    uint64_t last_stop_epoch;
 
     /* Device memory for kernels that split their work and merge it (zeroed
      * at creation; NULL and 0 when it could not be allocated). */
@@ -70,8 +73,8 @@ struct backend_kernel_s {
 };
 
 struct backend_encoder_s {
-    void*   ev_start;      /* hipEvent_t */
-    void*   ev_stop;       /* hipEvent_t */
+    void*   ev_start;      /* counted event (hip_backend.cpp) */
+    void*   ev_stop;       /* counted event */
     struct backend_ctx_s* ctx;
     uint64_t commit_epoch;
     int     committed;

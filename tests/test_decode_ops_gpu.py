@@ -24,6 +24,32 @@ def f32(*a):
     return np.array(a, np.float32)
 
 
+@pytest.mark.parametrize("order", [(0, 1, 2, 3), (3, 2, 1, 0), (2, 0, 3, 1)])
+def test_encoders_in_flight(be, order):
+    """Encoders committed behind one another (the next starts at the last one's stop event), waited for in any order,
+    and one begun on the idle stream: each reports its own GPU time, not the others'."""
+    n = 256 << 20
+    src, sink, p = be.alloc(n), be.alloc(16 * 4096), be.params(n, 4096, dtype=np.int64)
+    k = be.kernel("stream_read")
+    reps = (4, 1, 12, 4)
+
+    def commit(r):
+        enc = be.encoder()
+        for _ in range(r):
+            assert enc.dispatch(k, [src, sink, p], (4096 * 256,), (256,)) == 0
+        enc.commit()
+        return enc
+
+    commit(4).wait_timed()
+    be.synchronize()
+    encs = [commit(r) for r in reps]
+    ms = {i: encs[i].wait_timed() for i in order}
+    alone = commit(4).wait_timed()
+    # launches of one kernel: the reads of 256 MB take the same time each to well within a factor of two and a half
+    for i, r in enumerate(reps):
+        assert 0.4 * alone / 4 < ms[i] / r < 2.5 * alone / 4, (ms, alone)
+
+
 @pytest.mark.parametrize("N,C", [(1, 576), (3, 960), (2, 7), (1, 4096)])
 def test_rmsnorm_forward_v2(be, N, C):
     rng = np.random.default_rng(N * C)
