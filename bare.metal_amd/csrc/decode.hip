@@ -30,6 +30,7 @@
 #include "decode_state.h"
 #include "q8_common.h"
 #include "q8_gemm.h"
+#include "attn_prefill.h"
 #include "rows_gemm.h"
 
 #include <math.h>
@@ -1543,46 +1544,7 @@ __global__ __launch_bounds__(NT) void k_pf_attn(DecAttn a, const float* __restri
                        v + (size_t)p * a.KV + kh * HD);
 }
 
-/* Causal attention of a block of PQB = 16 consecutive prompt positions of
- * one query head, head size 64: softmax(q.k * scale) over keys 0..p, times
- * V, on fp32 MFMA (v_mfma_f32_16x16x4f32).  Two sources share the kernel:
- *  - PF_ENGINE: the engine's prefill.  q rows are un-roped ([n][NH*HD]; the
- *    kernel applies RoPE at each position as dec_attn_head does), K and V
- *    come from the KV cache of layer a.layer (K per KV head as
- *    [HD/4][MS] float4, V row-major [MS][KV]), the output is bf16 (the
- *    o-projection's operand).
- *  - PF_FLAT: the reference's prefill attention ABI (forward.metal:1904-2114):
- *    Q roped [S][NH][HD], K and V [S][NKV][HD], fp32 output [S][NH][HD].
- * Keys are staged through LDS in chunks of PKC: K row-major [key][dim],
- * V transposed [dim][key] (rows padded by 4 floats, so the 16 rows a wave
- * reads at once fall in different banks).  The chunk is cut into 16-key
- * sub-blocks dealt round-robin to the waves; per sub-block a wave forms
- *   S^T (16 keys x 16 queries) = K_sb Q^T   (16 MFMAs over the 64 dims),
- * updates a per-query online softmax, and accumulates
- *   O^T (64 dims x 16 queries) += V_sb^T P^T (16 MFMAs).
- * The MFMA sums run over any order of their index, so both products use a
- * permuted one: in S^T, step s of lane group g (= lane/16) takes dimension
- * 16g + s (a lane reads 16 consecutive dims of its key); in O^T, step s of
- * lane group g takes key 4g + s, which is exactly the key whose score that
- * lane holds in element s of its S^T fragment, so P^T goes from the score
- * registers to the next MFMA with no data movement.  Each wave's (max,
- * sum, O^T) is merged across waves through LDS at the end.  Keys at or
- * past n are staged as zeros, masked keys score -inf.  The summation order
- * differs from the one-query kernels; the mathematics is the same. */
-constexpr int PQB = 16;  /* prompt positions per workgroup */
-#ifndef PF_KCHUNK
-#define PF_KCHUNK 128
-#endif
-#ifndef PF_WAVES
-#define PF_WAVES 8
-#endif
-constexpr int PKC = PF_KCHUNK; /* keys per LDS chunk: one 16-key sub-block per wave and chunk */
-constexpr int PNW = PF_WAVES;  /* waves per workgroup: 8 (two per SIMD, one's softmax beside the other's
-                                  products) 15.4 us per layer at 512 tokens, 4 waves 18.3 us, 2 waves 27 */
-static_assert(PKC == 16 * PNW, "one 16-key sub-block per wave and chunk");
-constexpr int PNT = 64 * PNW;
-enum { PF_ENGINE = 0, PF_FLAT = 1 };
-
+/* The reference's prefill attention ABI. */
 struct PfFlat {
     const float* Q;
     const float* K;
@@ -1591,231 +1553,6 @@ struct PfFlat {
     float scale;
     int NH, S, NKV, kv_mul;
 };
-
-template <int MODE>
-__device__ __forceinline__ void pf_attn_block(const DecAttn& a, const PfFlat& f, const float* __restrict__ q,
-                                              unsigned short* __restrict__ out16, int n, int q_roped) {
-    constexpr int HD = 64, HD4 = HD / 4;
-    constexpr int LDK = HD + 4, LDVT = PKC + 4;
-    constexpr int NSB = PKC / 16; /* sub-blocks per chunk */
-    __shared__ float Ks[PKC * LDK];   /* [key][dim] */
-    __shared__ float Vt[HD * LDVT];   /* [dim][key] */
-    __shared__ float Qs[PQB * HD];    /* roped q of the block */
-    __shared__ float Ms[PNW * PQB], Ls[PNW * PQB];
-    const int NH = MODE == PF_FLAT ? f.NH : a.NH;
-    const int kv_mul = MODE == PF_FLAT ? f.kv_mul : a.NH / a.NKV;
-    /* scores in base 2: softmax weights by v_exp_f32 (exp2) of
-     * s * scale * log2(e), one instruction instead of expf's reduction */
-    const float sl2 = (MODE == PF_FLAT ? f.scale : a.scale) * 1.44269504088896341f;
-    /* the last blocks of the prompt have the most keys: they take the first
-     * workgroup slots, and the short ones fill in behind them */
-    const int h = blockIdx.x, p0 = (int)(gridDim.y - 1 - blockIdx.y) * PQB;
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-    const int col = lane & 15, grp = lane >> 4; /* MFMA column (query / key row) and lane group */
-    const int kh = h / kv_mul;
-    const int p = p0 + col; /* this lane's query position */
-    if (MODE == PF_FLAT || q_roped) { /* q already rotated */
-        const float* Q = MODE == PF_FLAT ? f.Q : q;
-        for (int i = t; i < PQB * HD; i += PNT) {
-            const int r = i / HD, e = i - r * HD;
-            Qs[i] = Q[((size_t)min(p0 + r, n - 1) * NH + h) * HD + e];
-        }
-    } else {
-        for (int i = t; i < PQB * (HD / 2); i += PNT) {
-            const int r = i / (HD / 2), e = i - r * (HD / 2);
-            const int pp = min(p0 + r, n - 1);
-            const float ang = (float)pp * a.inv_freq[e];
-            const float c = cosf(ang), sn = sinf(ang);
-            const size_t qr = (size_t)pp * NH * HD + h * HD;
-            const float q0 = q[qr + e];
-            const float q1 = q[qr + e + HD / 2];
-            Qs[r * HD + e] = q0 * c - q1 * sn;
-            Qs[r * HD + e + HD / 2] = q0 * sn + q1 * c;
-        }
-    }
-    __syncthreads();
-    /* Q^T fragment: step s holds q[col][16*grp + s] */
-    float qf[16];
-#pragma unroll
-    for (int s = 0; s < 16; s++) qf[s] = Qs[col * HD + 16 * grp + s];
-    bmv_f32x4 acc[4]; /* O^T tile t: dims 16t + 4*grp + v, query col */
-#pragma unroll
-    for (int i = 0; i < 4; i++) acc[i] = bmv_f32x4{0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.0f; /* m: per query (same in the 4 lane groups); l: this lane's keys */
-    /* K source: dims 4g..4g+3 of key j at ksrc + j * kstr + g * kgstr (floats); V: row j at vsrc + j * vstr */
-    const float *ksrc, *vsrc;
-    size_t kstr, kgstr, vstr;
-    if (MODE == PF_FLAT) {
-        const size_t KVW = (size_t)f.NKV * HD;
-        ksrc = f.K + kh * HD;
-        kstr = KVW;
-        kgstr = 4;
-        vsrc = f.V + kh * HD;
-        vstr = KVW;
-    } else {
-        const size_t slab = (size_t)a.MS * a.KV;
-        ksrc = a.kvc + (size_t)a.layer * 2 * slab + (size_t)kh * HD * a.MS;
-        kstr = 4;
-        kgstr = (size_t)a.MS * 4;
-        vsrc = a.kvc + ((size_t)a.layer * 2 + 1) * slab + kh * HD;
-        vstr = a.KV;
-    }
-    /* Chunk staging: each thread moves SPT float4 of K (element i: dims
-     * 4*(i / PKC), key i % PKC, so a wave reads consecutive keys of one
-     * cache row) and of V (element i = 64 w + l: keys 16 (w % 4) + l % 16,
-     * dims 4 (4 (w / 4) + l / 16): a wave instruction covers 16 keys x 16
-     * dims, so its transposed writes into Vt fall in distinct banks; with
-     * whole rows per instruction they conflicted 8 ways, 0.7 us per chunk).
-     * The loads of chunk c+1 are issued into registers before chunk c is
-     * computed, unconditionally (key clamped to n-1; keys at or past n
-     * become zeros when written to LDS). */
-    constexpr int SPT = PKC * HD4 / PNT;
-    static_assert(HD4 == 16 && PKC % 16 == 0, "V staging map: 16 dim groups, 16-key runs");
-    auto vkey = [](int i) { return 16 * ((i >> 6) % (PKC / 16)) + (i & 15); };
-    auto vgrp = [](int i) { return 4 * ((i >> 6) / (PKC / 16)) + ((i & 63) >> 4); };
-    float4 kreg[SPT], vreg[SPT];
-    auto fetch = [&](int c0) {
-#pragma unroll
-        for (int u = 0; u < SPT; u++) {
-            const int i = t + PNT * u;
-            const int kk = min(c0 + i % PKC, n - 1), kg = i / PKC;
-            const int vk = min(c0 + vkey(i), n - 1), vg = vgrp(i);
-            __builtin_memcpy(&kreg[u], __builtin_assume_aligned(ksrc + (size_t)kk * kstr + kg * kgstr, 16), 16);
-            __builtin_memcpy(&vreg[u], __builtin_assume_aligned(vsrc + (size_t)vk * vstr + 4 * vg, 16), 16);
-        }
-    };
-    const int kend = min(p0 + PQB, n); /* keys 0 .. kend-1 */
-    fetch(0);
-    for (int c0 = 0; c0 < kend; c0 += PKC) {
-        __syncthreads(); /* the previous chunk has been read */
-#pragma unroll
-        for (int u = 0; u < SPT; u++) {
-            const int i = t + PNT * u;
-            const int kk = i % PKC, kg = i / PKC, vk = vkey(i), vg = vgrp(i);
-            const bool kin = c0 + kk < n, vin = c0 + vk < n;
-            const float4 kv = kreg[u], vv = vreg[u];
-            *(float4*)&Ks[kk * LDK + 4 * kg] =
-                make_float4(kin ? kv.x : 0.f, kin ? kv.y : 0.f, kin ? kv.z : 0.f, kin ? kv.w : 0.f);
-            Vt[(4 * vg + 0) * LDVT + vk] = vin ? vv.x : 0.f;
-            Vt[(4 * vg + 1) * LDVT + vk] = vin ? vv.y : 0.f;
-            Vt[(4 * vg + 2) * LDVT + vk] = vin ? vv.z : 0.f;
-            Vt[(4 * vg + 3) * LDVT + vk] = vin ? vv.w : 0.f;
-        }
-        __syncthreads();
-        if (c0 + PKC < kend) fetch(c0 + PKC);
-        for (int sb = wave; sb < NSB; sb += PNW) {
-            const int k0 = c0 + 16 * sb; /* first key of the sub-block */
-            if (k0 >= kend) break;       /* past every query of the block (wave-uniform) */
-            /* S^T[key 4*grp + v][query col] */
-            /* four independent chains over the 64 dimensions (a single
-             * chain of 16 dependent MFMAs waits out each one's latency) */
-            bmv_f32x4 sq[4];
-            const float* kr = &Ks[(16 * sb + col) * LDK + 16 * grp];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float4 k4 = *(const float4*)&kr[4 * i];
-                sq[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.x, qf[4 * i + 0], bmv_f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float4 k4 = *(const float4*)&kr[4 * i];
-                sq[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.y, qf[4 * i + 1], sq[i], 0, 0, 0);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float4 k4 = *(const float4*)&kr[4 * i];
-                sq[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.z, qf[4 * i + 2], sq[i], 0, 0, 0);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float4 k4 = *(const float4*)&kr[4 * i];
-                sq[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.w, qf[4 * i + 3], sq[i], 0, 0, 0);
-            }
-            const bmv_f32x4 st = (sq[0] + sq[1]) + (sq[2] + sq[3]);
-            float sv[4];
-            float cm = -INFINITY;
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                sv[v] = k0 + 4 * grp + v <= p ? st[v] * sl2 : -INFINITY;
-                cm = fmaxf(cm, sv[v]);
-            }
-            cm = fmaxf(cm, __shfl_xor(cm, 16));
-            cm = fmaxf(cm, __shfl_xor(cm, 32));
-            const float mn = fmaxf(m, cm);
-            const bool live = mn > -INFINITY; /* some key of this query admitted so far */
-            const float fr = live ? __builtin_amdgcn_exp2f(m - mn) : 1.0f;
-            float pv[4];
-#pragma unroll
-            for (int v = 0; v < 4; v++) pv[v] = live ? __builtin_amdgcn_exp2f(sv[v] - mn) : 0.0f;
-            l = l * fr + ((pv[0] + pv[1]) + (pv[2] + pv[3]));
-#pragma unroll
-            for (int ti = 0; ti < 4; ti++) acc[ti] *= fr;
-            m = live ? mn : m;
-            /* O^T[dim 16t + col'][query] += V^T[dim][key 4*grp + s] * P^T[key][query] */
-#pragma unroll
-            for (int ti = 0; ti < 4; ti++) {
-                const float4 v4 = *(const float4*)&Vt[(16 * ti + col) * LDVT + 16 * sb + 4 * grp];
-                acc[ti] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.x, pv[0], acc[ti], 0, 0, 0);
-                acc[ti] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.y, pv[1], acc[ti], 0, 0, 0);
-                acc[ti] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.z, pv[2], acc[ti], 0, 0, 0);
-                acc[ti] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.w, pv[3], acc[ti], 0, 0, 0);
-            }
-        }
-    }
-    /* this wave's sum over its keys: add the four lane groups */
-    l += __shfl_xor(l, 16);
-    l += __shfl_xor(l, 32);
-    __syncthreads(); /* every wave is done with Ks */
-    float* Ws = Ks; /* [wave][dim][query] */
-#pragma unroll
-    for (int ti = 0; ti < 4; ti++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) Ws[(wave * HD + 16 * ti + 4 * grp + v) * PQB + col] = acc[ti][v];
-    if (grp == 0) {
-        Ms[wave * PQB + col] = m;
-        Ls[wave * PQB + col] = l;
-    }
-    __syncthreads();
-    const int r = t / HD4, g = t - r * HD4; /* query r, dimensions 4g .. 4g+3 */
-    if (r >= PQB || p0 + r >= n) return;
-    float mx = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < PNW; w++) mx = fmaxf(mx, Ms[w * PQB + r]);
-    float den = 0.f, o0 = 0.f, o1 = 0.f, o2 = 0.f, o3 = 0.f;
-#pragma unroll
-    for (int w = 0; w < PNW; w++) {
-        const float mv = Ms[w * PQB + r];
-        const float fr = mv == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mv - mx);
-        const float* src = &Ws[(w * HD + 4 * g) * PQB + r];
-        den = fmaf(fr, Ls[w * PQB + r], den);
-        o0 = fmaf(fr, src[0 * PQB], o0);
-        o1 = fmaf(fr, src[1 * PQB], o1);
-        o2 = fmaf(fr, src[2 * PQB], o2);
-        o3 = fmaf(fr, src[3 * PQB], o3);
-    }
-    const size_t off = ((size_t)(p0 + r) * NH + h) * HD + 4 * g;
-    if (MODE == PF_FLAT) {
-        f.out[off + 0] = o0 / den;
-        f.out[off + 1] = o1 / den;
-        f.out[off + 2] = o2 / den;
-        f.out[off + 3] = o3 / den;
-    } else { /* the o projection's operand: fragment order, four consecutive values */
-        const uint2 o = make_uint2((unsigned int)bf16_bits(o0 / den) | ((unsigned int)bf16_bits(o1 / den) << 16),
-                                   (unsigned int)bf16_bits(o2 / den) | ((unsigned int)bf16_bits(o3 / den) << 16));
-        *(uint2*)(out16 + frag_index(p0 + r, h * HD + 4 * g, (NH * HD + 63) >> 6)) = o;
-    }
-}
-
-__global__ __launch_bounds__(PNT) void k_pf_attn_blk(DecAttn a, const float* __restrict__ q,
-                                                    unsigned short* __restrict__ out16, int n, int q_roped) {
-    const PfFlat f = {};
-    pf_attn_block<PF_ENGINE>(a, f, q, out16, n, q_roped);
-}
-
-__global__ __launch_bounds__(PNT) void k_attn_prefill64(PfFlat f) {
-    const DecAttn a = {};
-    pf_attn_block<PF_FLAT>(a, f, nullptr, nullptr, f.S, 0);
-}
 
 /* Any head size up to 128 on the reference's prefill attention ABI: one
  * wave per (query position, head); lane owns dimensions lane and lane + 64;
@@ -1995,10 +1732,11 @@ extern "C" int bmk_launch_attention_prefill(const bmk_launch_t* a) {
     f.V = (const float*)a->dev[2];
     f.out = (float*)a->dev[3];
     const bool aligned = (((uintptr_t)a->dev[0] | (uintptr_t)a->dev[1] | (uintptr_t)a->dev[2] | (uintptr_t)a->dev[3]) & 15) == 0;
-    if (HD == 64 && aligned)
-        hipLaunchKernelGGL(k_attn_prefill64, dim3(f.NH, (f.S + PQB - 1) / PQB), dim3(PNT), 0, a->stream, f);
-    else
-        hipLaunchKernelGGL(k_attn_prefill_wave, dim3(f.NH, (f.S + 3) / 4), dim3(NT), 0, a->stream, f, HD);
+    if (HD == 64 && aligned) {
+        const ApArgs p = {f.Q, f.K, f.V, f.out, nullptr, f.NH, f.S, f.kv_mul, f.NKV * HD, 0, f.scale};
+        return ap_launch(&p, 0, a->stream);
+    }
+    hipLaunchKernelGGL(k_attn_prefill_wave, dim3(f.NH, (f.S + 3) / 4), dim3(NT), 0, a->stream, f, HD);
     BMK_LAUNCH_CHECK();
     return 0;
 }
@@ -2431,10 +2169,10 @@ extern "C" int dec_pf_attention(const DecAttn* a, const float* q, const float* k
         BMK_LAUNCH_CHECK();
     }
     if (a->HD == 64) {
-        hipLaunchKernelGGL(k_pf_attn_blk, dim3(a->NH, (n + PQB - 1) / PQB), dim3(PNT), 0, s, *a, q, out16, n,
-                           kv_done);
-        BMK_LAUNCH_CHECK();
-        return 0;
+        const size_t slab = (size_t)a->MS * a->KV;
+        const float* kc = a->kvc + (size_t)a->layer * 2 * slab;
+        const ApArgs p = {q, kc, kc + slab, nullptr, out16, a->NH, n, a->NH / a->NKV, a->KV, a->MS, a->scale};
+        return ap_launch(&p, 1, s);
     }
     const dim3 g(a->NH, n);
     if (a->HD == 128) hipLaunchKernelGGL(k_pf_attn<128>, g, dim3(NT), 0, s, *a, q, k, v);

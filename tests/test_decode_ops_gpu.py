@@ -303,6 +303,30 @@ def test_attention_prefill_equal_keys_is_running_mean(be, HD):
     assert nw(out.read(np.float32), want) <= TOL
 
 
+@pytest.mark.parametrize("S", [1, 15, 16, 17, 64, 65, 127, 130, 145, 300])
+@pytest.mark.parametrize("NH,NKV", [(3, 1), (4, 4)])
+def test_attention_prefill_sub_blocks(be, S, NH, NKV):
+    """Prompts whose last 16-key sub-block is partly filled and whose waves take one, two or several sub-blocks each,
+    scores that climb so far that the running maximum has to move (and fall so far that it must not), with memory
+    past the prompt's rows NaN; fp32 sums against 64 bits."""
+    HD = 64
+    rng = np.random.default_rng(S)
+    Q = rng.standard_normal(S * NH * HD).astype(np.float32)
+    K = (rng.standard_normal((S, NKV, HD)) * np.linspace(0.2, 6.0, S)[:, None, None]).astype(np.float32)
+    K[S // 2:] *= 0.3
+    V = rng.standard_normal(S * NKV * HD).astype(np.float32)
+    nan = np.full(64 * HD, np.nan, np.float32)
+    out = be.upload(np.full(S * NH * HD + 64, 5.0, np.float32))
+    bufs = [be.upload(np.concatenate([x.ravel(), nan])) for x in (Q, K, V)]
+    assert be.dispatch("attention_forward_prefill", bufs + [out, be.params(NH, S, HD, NKV, NH // NKV),
+                                                           be.upload(f32(0.25))], (NH * S,), (256,)) == 0
+    got = out.read(np.float32)
+    want = prefill_attn_ref(Q, K.ravel(), V, NH, NKV, HD, S, NH // NKV, np.float32(0.25))
+    # scores reach about 0.25 * 64 * 6 / 3 = 30 in base e: their fp32 rounding moves a weight by 30 * 2^-23 = 4e-6
+    assert nw(got[:S * NH * HD], want) <= TOL
+    assert (got[S * NH * HD:] == 5.0).all()
+
+
 def test_attention_prefill_rejects(be):
     NH, NKV, HD, S = 4, 2, 64, 8
     Q = np.zeros(S * NH * HD, np.float32)
