@@ -84,17 +84,29 @@ __device__ __forceinline__ Blk4 zero_block4() {
 /* code k (0..7) of a dword of packed nibbles, exactly as fp32 */
 __device__ __forceinline__ float q4_code(unsigned int w, int k) { return (float)((int)(w << (28 - 4 * k)) >> 28); }
 
-__device__ __forceinline__ float dot8_q4(unsigned int w, const float* x) {
-    float a = x[0] * q4_code(w, 0);
+/* One sixteenth of the product of a dword's codes with x.
+ * v_cvt_off_f32_i4 turns the low nibble of the byte that its operand selects
+ * into code / 16 exactly, so eight codes cost eight conversions and one shift
+ * (sign extension and conversion cost two instructions a code).  The empty
+ * asm keeps the shifted dword whole: merged with the byte selection the shift
+ * becomes an instruction of its own for every high nibble. */
+__device__ __forceinline__ float dot8_q4_16(unsigned int w, const float* x) {
+    unsigned int hi = w >> 4;
+    asm("" : "+v"(hi));
+    float a = x[0] * __builtin_amdgcn_cvt_off_f32_i4((int)(w & 0xffu));
+    a = fmaf(x[1], __builtin_amdgcn_cvt_off_f32_i4((int)(hi & 0xffu)), a);
 #pragma unroll
-    for (int k = 1; k < 8; k++) a = fmaf(x[k], q4_code(w, k), a);
+    for (int k = 1; k < 4; k++) {
+        a = fmaf(x[2 * k], __builtin_amdgcn_cvt_off_f32_i4((int)((w >> (8 * k)) & 0xffu)), a);
+        a = fmaf(x[2 * k + 1], __builtin_amdgcn_cvt_off_f32_i4((int)((hi >> (8 * k)) & 0xffu)), a);
+    }
     return a;
 }
 
 __device__ __forceinline__ float block_dot(const Blk4& b, const float* xs) {
-    const float s0 = dot8_q4(b.q.x, xs + 0) + dot8_q4(b.q.y, xs + 8);
-    const float s1 = dot8_q4(b.q.z, xs + 16) + dot8_q4(b.q.w, xs + 24);
-    return (s0 + s1) * b.s;
+    const float s0 = dot8_q4_16(b.q.x, xs + 0) + dot8_q4_16(b.q.y, xs + 8);
+    const float s1 = dot8_q4_16(b.q.z, xs + 16) + dot8_q4_16(b.q.w, xs + 24);
+    return ((s0 + s1) * 16.0f) * b.s;
 }
 
 /* Block formats of the quantized kernels: bytes per 32-weight block and the
