@@ -24,8 +24,15 @@
  *    engine makes once per model).  Scattered 16-byte loads (32 rows per
  *    instruction) cost 2.7-4.8 us more per launch at 512 tokens;
  *  - the four waves of a workgroup split K (contiguous step ranges), with
- *    the loads of three steps in flight, and sum their partial tiles through
- *    LDS once at the end, in wave order (the same bits every run);
+ *    the loads of three steps in flight throughout (refilled step by step;
+ *    in groups of three, each group exposed a whole latency), and sum their
+ *    partial tiles through LDS once at the end, in wave order (the same bits
+ *    every run);
+ *  - the first steps' loads go out before the epilogue's inputs, which loads
+ *    return behind them: with those first, and conditional, the first products
+ *    waited for them.  With the refill: a prompt's pass of 16 / 128 / 512 / 2000
+ *    tokens, 135M 824 -> 771, 884 -> 850, 1267 -> 1272, 3850 -> 3690 us; 360M 1180 ->
+ *    1080, 1276 -> 1190, 2051 -> 1990, 6850 -> 6400 us;
  *  - the consumer runs in the epilogue: the plain store, the q/k/v
  *    epilogue (k rotated by RoPE and appended to the KV cache with v, as
  *    the reference's rope and cache-append kernels do, forward.metal:1284-
@@ -71,16 +78,30 @@ __device__ __forceinline__ float sb(unsigned int w, int k) { return (float)(sign
  * groups (32 bf16 each) and its weight block in both column groups. */
 template <int QF, int MI, int NJ>
 struct PfgStage {
-    uint4 a[MI][4];
+    u32x4 a[MI][4];
     float s[NJ];
-    uint4 q[NJ][QF == QF_Q4 ? 1 : 2];
+    u32x4 q[NJ][QF == QF_Q4 ? 1 : 2];
 };
+
+/* Keeps what is computed from a loaded value behind this point: hoisted
+ * ahead of the loop's next step it would wait for loads just issued, and hold
+ * the converted values in registers instead of the codes. */
+template <class T>
+__device__ __forceinline__ void pin(T& v) { asm volatile("" : "+v"(v)); }
+
+/* 16 bytes from an address aligned to AL */
+template <int AL>
+__device__ __forceinline__ u32x4 ld16(const void* p) {
+    u32x4 v;
+    __builtin_memcpy(&v, __builtin_assume_aligned(p, AL), 16);
+    return v;
+}
 
 /* Codes 8u .. 8u+7 of a block, times its scale, rounded to bf16. */
 template <int QF>
-__device__ __forceinline__ bf16x8 dq(const uint4* q, int u, float s) {
+__device__ __forceinline__ bf16x8 dq(const u32x4* q, int u, float s) {
     unsigned int w0, w1;
-    uint4 r;
+    u32x4 r;
     if (QF == QF_Q4) {
         const unsigned int w = u == 0 ? q[0].x : u == 1 ? q[0].y : u == 2 ? q[0].z : q[0].w;
         r.x = pk2(q4_code(w, 0) * s, q4_code(w, 1) * s);
@@ -88,7 +109,7 @@ __device__ __forceinline__ bf16x8 dq(const uint4* q, int u, float s) {
         r.z = pk2(q4_code(w, 4) * s, q4_code(w, 5) * s);
         r.w = pk2(q4_code(w, 6) * s, q4_code(w, 7) * s);
     } else {
-        const uint4& h = q[u >> 1];
+        const u32x4 h = q[u >> 1];
         w0 = (u & 1) ? h.z : h.x;
         w1 = (u & 1) ? h.w : h.y;
         r.x = pk2(sb(w0, 0) * s, sb(w0, 1) * s);
@@ -96,9 +117,7 @@ __device__ __forceinline__ bf16x8 dq(const uint4* q, int u, float s) {
         r.z = pk2(sb(w1, 0) * s, sb(w1, 1) * s);
         r.w = pk2(sb(w1, 2) * s, sb(w1, 3) * s);
     }
-    bf16x8 b;
-    __builtin_memcpy(&b, &r, 16);
-    return b;
+    return __builtin_bit_cast(bf16x8, r);
 }
 
 template <int QF, int EPI, int MI, int NJ>
@@ -110,7 +129,7 @@ __global__ __launch_bounds__(PNTH) void k_pf_gemm(PfgArgs a) {
     __shared__ float part[4][PTM][TW + 4];
     __shared__ float sst[PFG_SS_MAX][PT]; /* the tile rows' partial sums of squares */
     constexpr unsigned CH = QF == QF_Q4 ? PFG_CHUNK_Q4 : PFG_CHUNK_Q8;
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
     const int col = lane & 31, h = lane >> 5;
     const int nt = (int)(blockIdx.x % (unsigned)a.NT), mt = (int)(blockIdx.x / (unsigned)a.NT);
     const int M = a.M, ns = (a.K + 63) >> 6; /* 64-wide K steps (fragment columns per row block) */
@@ -131,7 +150,7 @@ __global__ __launch_bounds__(PNTH) void k_pf_gemm(PfgArgs a) {
 #pragma unroll
     for (int i = 0; i < MI; i++) {
         const int rb = min((m0 >> 5) + i, ((M + 31) >> 5) - 1);
-        af[i] = a.A + (size_t)rb * ns * 2048 + 8 * lane;
+        af[i] = a.A + (size_t)rb * ns * 2048;
     }
 #pragma unroll
     for (int i = 0; i < NJ; i++) {
@@ -139,6 +158,32 @@ __global__ __launch_bounds__(PNTH) void k_pf_gemm(PfgArgs a) {
         wc[i] = a.W + a.p[EPI == PFG_SWIGLU ? i : p].w_off + (size_t)f * ns * CH;
     }
     const int s_beg = wave * ns / 4, s_end = (wave + 1) * ns / 4;
+    const unsigned int o16 = 16u * (unsigned)lane; /* from wave-uniform bases: no address held per load */
+    auto load = [&](int s, PfgStage<QF, MI, NJ>& st) { /* past the wave's last step: that step again */
+        s = max(min(s, s_end - 1), 0);
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                st.a[i][u] = ld16<16>((const char*)(af[i] + (size_t)s * 2048) + (o16 + 1024u * u));
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            const unsigned char* c = wc[j] + (size_t)s * CH;
+            st.s[j] = *(const float*)(c + 4u * (unsigned)lane);
+            st.q[j][0] = ld16<16>(c + (o16 + 256u));
+            if (QF == QF_Q8) st.q[j][QF == QF_Q8 ? 1 : 0] = ld16<16>(c + (o16 + 1280u));
+        }
+    };
+    /* The first three steps' operands are on their way before anything that
+     * only the epilogue reads: loads return in order, and the K loop's first
+     * wait must not be for those. */
+    PfgStage<QF, MI, NJ> s0, s1, s2;
+    load(s_beg, s0);
+    __builtin_amdgcn_sched_barrier(0);
+    load(s_beg + 1, s1);
+    __builtin_amdgcn_sched_barrier(0);
+    load(s_beg + 2, s2);
+    __builtin_amdgcn_sched_barrier(0);
     /* Epilogue thread map: row r of the tile; CPT columns from c0 (8 gate
      * and 8 up columns from j0 for SwiGLU). */
     const int r = t >> 2, m = m0 + r, c0 = (t & 3) * CPT, j0 = (t & 3) * 8;
@@ -149,44 +194,36 @@ __global__ __launch_bounds__(PNTH) void k_pf_gemm(PfgArgs a) {
                                          : nullptr);
     const bool whole = (EPI == PFG_STORE || EPI == PFG_RESID || (EPI == PFG_QKV && p == 0)) && n0 + c0 + CPT <= N &&
                        ((uintptr_t)dst & 15) == 0;
-    /* the residual rows this thread adds to, loaded before the K loop so
-     * that their latency hides behind it */
-    float4 res[CPT / 4];
-    if (EPI == PFG_RESID && whole && r < PTM) {
+    /* What the epilogue reads, loaded ahead of the K loop.  A launch with a
+     * residual: its rows and, when it writes the next norm's operand, that
+     * norm's weights; a thread's CPT columns lie inside N or past it (N is a
+     * multiple of 32), and past it the last ones are read for nothing. */
+    f32x4 res[CPT / 4], gnr[CPT / 4];
+    if (EPI == PFG_RESID) {
+        const int cc = max(min(n0 + c0, N - CPT), 0);
+        const float* rp = a.x + (size_t)min(m, M - 1) * ldc + cc;
+        const float* gp = a.an ? a.gn + cc : rp; /* no branch around a load: the waits would be for the worse case */
 #pragma unroll
-        for (int c = 0; c < CPT / 4; c++) res[c] = *(const float4*)&dst[4 * c];
+        for (int c = 0; c < CPT / 4; c++) res[c] = __builtin_bit_cast(f32x4, ld16<4>(rp + 4 * c));
+#pragma unroll
+        for (int c = 0; c < CPT / 4; c++) gnr[c] = __builtin_bit_cast(f32x4, ld16<4>(gp + 4 * c));
     }
-    /* The RMSNorm inputs, loaded before the K loop so that their latency
-     * hides behind it: the tile rows' partial sums of squares, straight
-     * into LDS (global_load_lds: one tile's 64 rows per wave instruction,
-     * no registers held across the loop), or, for a residual launch that
-     * writes the next norm's operand, the norm weights of its 16 columns. */
+    /* q/k/v: the position's (cos, sin) of this thread's eight rotary pairs */
+    f32x4 rt[4];
+    if (EPI == PFG_QKV) {
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+            rt[c] = __builtin_bit_cast(f32x4, ld16<16>(&a.rope[((size_t)min(m, M - 1) * 32 + j0 + 2 * c) * 2]));
+    }
+    /* the tile rows' partial sums of squares, straight into LDS
+     * (global_load_lds: one tile's 64 rows per wave instruction, no registers
+     * held across the loop) */
     if (EPI != PFG_RESID && a.ss_in) {
         for (int i = wave; i < a.ss_tiles; i += 4)
             __builtin_amdgcn_global_load_lds(
                 (const __attribute__((address_space(1))) void*)(a.ss_in + (size_t)i * a.ss_ld + min(m0 + lane, M - 1)),
                 (__attribute__((address_space(3))) void*)&sst[i][0], 4, 0, 0);
     }
-    float gnr[CPT];
-    if (EPI == PFG_RESID && a.an && r < PTM) {
-#pragma unroll
-        for (int c = 0; c < CPT; c++) gnr[c] = a.gn[min(n0 + c0 + c, N - 1)];
-    }
-
-    auto load = [&](int s, PfgStage<QF, MI, NJ>& st) {
-#pragma unroll
-        for (int i = 0; i < MI; i++)
-#pragma unroll
-            for (int u = 0; u < 4; u++)
-                __builtin_memcpy(&st.a[i][u], __builtin_assume_aligned(af[i] + (size_t)s * 2048 + 512 * u, 16), 16);
-#pragma unroll
-        for (int j = 0; j < NJ; j++) {
-            const unsigned char* c = wc[j] + (size_t)s * CH;
-            __builtin_memcpy(&st.s[j], __builtin_assume_aligned(c + 4 * lane, 4), 4);
-            __builtin_memcpy(&st.q[j][0], __builtin_assume_aligned(c + 256 + 16 * lane, 16), 16);
-            if (QF == QF_Q8) __builtin_memcpy(&st.q[j][QF == QF_Q8 ? 1 : 0], __builtin_assume_aligned(c + 1280 + 16 * lane, 16), 16);
-        }
-    };
 
     f32x16 acc[MI][NJ];
 #pragma unroll
@@ -198,14 +235,20 @@ __global__ __launch_bounds__(PNTH) void k_pf_gemm(PfgArgs a) {
 
     /* Past an odd block count the last step's upper half is zero on both
      * sides (the producers' column padding, the layout's zero blocks). */
-    auto compute = [&](const PfgStage<QF, MI, NJ>& st) {
+    auto compute = [&](PfgStage<QF, MI, NJ>& st) {
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            pin(st.s[j]);
+            pin(st.q[j][0]);
+            if (QF == QF_Q8) pin(st.q[j][QF == QF_Q8 ? 1 : 0]);
+        }
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             bf16x8 fb[NJ], fa[MI];
 #pragma unroll
             for (int j = 0; j < NJ; j++) fb[j] = dq<QF>(st.q[j], u, st.s[j]);
 #pragma unroll
-            for (int i = 0; i < MI; i++) __builtin_memcpy(&fa[i], &st.a[i][u], 16);
+            for (int i = 0; i < MI; i++) fa[i] = __builtin_bit_cast(bf16x8, st.a[i][u]);
 #pragma unroll
             for (int i = 0; i < MI; i++)
 #pragma unroll
@@ -214,19 +257,28 @@ __global__ __launch_bounds__(PNTH) void k_pf_gemm(PfgArgs a) {
         }
     };
 
-    /* Groups of three steps: all loads of a group are issued first (past
-     * the wave's last step they repeat it: an L2 hit, never used, so every
-     * path issues the same loads), then each step waits for its own. */
-    for (int g = s_beg; g < s_end; g += 3) {
-        PfgStage<QF, MI, NJ> s0, s1, s2;
-        load(g, s0);
-        load(min(g + 1, s_end - 1), s1);
-        load(min(g + 2, s_end - 1), s2);
-        __builtin_amdgcn_sched_barrier(0);
+    /* Three steps in registers; while more than three are left, each one's
+     * registers are refilled as soon as its products are issued (the
+     * scheduler, left alone, loads into others and copies, which waits for
+     * the loads). */
+    int step = s_beg;
+    for (; step + 3 < s_end; step += 3) {
         compute(s0);
-        if (g + 1 < s_end) compute(s1);
-        if (g + 2 < s_end) compute(s2);
+        __builtin_amdgcn_sched_barrier(0);
+        load(step + 3, s0);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(s1);
+        __builtin_amdgcn_sched_barrier(0);
+        load(step + 4, s1);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(s2);
+        __builtin_amdgcn_sched_barrier(0);
+        load(step + 5, s2);
+        __builtin_amdgcn_sched_barrier(0);
     }
+    if (step < s_end) compute(s0);
+    if (step + 1 < s_end) compute(s1);
+    if (step + 2 < s_end) compute(s2);
 
     /* Partial tiles to LDS (32x32 D layout: register r of a tile holds row
      * 8 (r / 4) + 4 h + r % 4, column l % 32), then the sum in wave order. */
@@ -307,7 +359,7 @@ __global__ __launch_bounds__(PNTH) void k_pf_gemm(PfgArgs a) {
         float cs[8], sn[8];
 #pragma unroll
         for (int c = 0; c < 8; c += 2) {
-            const float4 t4 = *(const float4*)&a.rope[((size_t)m * 32 + j0 + c) * 2];
+            const f32x4 t4 = rt[c >> 1];
             cs[c] = t4.x; sn[c] = t4.y; cs[c + 1] = t4.z; sn[c + 1] = t4.w;
         }
         float* kT = a.kc + (size_t)(n0 >> 6) * 64 * a.MS;
@@ -345,7 +397,7 @@ __global__ __launch_bounds__(PNTH) void k_pf_gemm(PfgArgs a) {
             float vv[4] = {v.x, v.y, v.z, v.w};
             if (whole) {
                 if (EPI == PFG_RESID) {
-                    const float4 o = res[c >> 2];
+                    const f32x4 o = res[c >> 2];
                     vv[0] += o.x; vv[1] += o.y; vv[2] += o.z; vv[3] += o.w;
                 }
                 const f32x4 v4 = {vv[0], vv[1], vv[2], vv[3]};
@@ -379,8 +431,8 @@ __global__ __launch_bounds__(PNTH) void k_pf_gemm(PfgArgs a) {
 #pragma unroll
                 for (int c = 0; c < 8; c += 2) {
                     const int cc = n0 + c0 + 8 * hf + c;
-                    const float lo = cc < N ? xn[8 * hf + c] * gnr[8 * hf + c] : 0.f;
-                    const float hi = cc + 1 < N ? xn[8 * hf + c + 1] * gnr[8 * hf + c + 1] : 0.f;
+                    const float lo = cc < N ? xn[8 * hf + c] * gnr[(8 * hf + c) >> 2][c & 3] : 0.f;
+                    const float hi = cc + 1 < N ? xn[8 * hf + c + 1] * gnr[(8 * hf + c + 1) >> 2][(c + 1) & 3] : 0.f;
                     w[c >> 1] = pk2(lo, hi);
                 }
                 *(uint4*)(a.an + frag_index(m, n0 + c0 + 8 * hf, nks)) = make_uint4(w[0], w[1], w[2], w[3]);
