@@ -64,6 +64,24 @@ def test_rmsnorm_forward_v2(be, N, C):
     assert nw(out.read(np.float32), want.ravel()) <= TOL
 
 
+@pytest.mark.parametrize("N,C,off", [(5, 4, 0), (2, 1020, 0), (3, 1024, 0), (3, 1028, 0), (2, 4096, 0), (2, 4100, 0),
+                                     (4, 576, 4), (3, 962, 0)])
+@pytest.mark.parametrize("inplace", [False, True])
+def test_rmsnorm_forward_v2_groups(be, N, C, off, inplace):
+    """Row lengths around the 16-byte form's (1024 and 4096 at most), rows that are not whole groups, operands that are
+    not 16-byte aligned, and the input as the output; fp32 sums against 64 bits."""
+    rng = np.random.default_rng(N * C + off)
+    x = rng.standard_normal(N * C + off // 4).astype(np.float32)
+    w = rng.uniform(0.5, 1.5, C).astype(np.float32)
+    bx = be.upload(x)
+    out = bx if inplace else be.alloc(N * C * 4 + off)
+    assert be.dispatch("rmsnorm_forward_v2", [bx, be.upload(w), out, be.params(N, C), be.upload(f32(1e-5))], (256,),
+                       (256,), offsets=[off, 0, off, 0, 0]) == 0
+    xr = x[off // 4:].reshape(N, C).astype(np.float64)
+    want = xr / np.sqrt((xr * xr).mean(axis=1, keepdims=True) + 1e-5) * w
+    assert nw(out.read(np.float32, N * C, off), want.ravel()) <= TOL
+
+
 _libm = ctypes.CDLL("libm.so.6")
 _libm.powf.restype = ctypes.c_float
 _libm.powf.argtypes = [ctypes.c_float, ctypes.c_float]
