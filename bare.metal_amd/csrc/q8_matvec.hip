@@ -89,7 +89,15 @@ __device__ __forceinline__ void mv_tile(const MvProb& p, int tile, float* red) {
         if (r < p.OC) {
             const float* rp = red + rl * nb;
             float acc = 0.0f;
-            for (int k = 0; k < nb; k++) acc += rp[k];
+            int k = 0;
+            for (; k + 8 <= nb; k += 8) { /* eight LDS reads in flight, added in block order */
+                float v[8];
+#pragma unroll
+                for (int e = 0; e < 8; e++) v[e] = rp[k + e];
+#pragma unroll
+                for (int e = 0; e < 8; e++) acc += v[e];
+            }
+            for (; k < nb; k++) acc += rp[k];
             if (p.bias) acc += p.bias[r];
             p.y[r] = acc;
         }
@@ -646,15 +654,28 @@ extern "C" int mv_tiles_for(int OC, int C, int U) {
  * roofline; fewer, wider tiles would starve the CUs on small matrices.
  * Measured on the 49152-row LM heads, launch after launch over weights no
  * cache holds: 12.9 us at 8 rows per lane against 14.1 at 4 (x960), 9.5
- * against 9.8 (x576); 1 or 2 rows per lane are slower, 16 too. */
+ * against 9.8 (x576); 1 or 2 rows per lane are slower, 16 too.
+ * At the other end a launch is one workgroup's chain, and rows in flight
+ * only lengthen it: one row per lane where that fills at most one workgroup
+ * per CU, else two.  Back to back, 4 rows / now (us): 576 x 576 4.07 / 3.45, 1536 x
+ * 576 4.08 / 3.41, 576 x 1536 4.35 / 3.51, 960 x 960 4.22 / 3.52, 2560 x 960 (two rows) 4.21
+ * / 3.85, 960 x 2560 4.45 / 3.89; one row there, 320 workgroups, 4.46. */
 #define MV_WIDE_MIN_TILES 768
+#define MV_CUS 256
 
 template <int QF>
 static int launch_group(MvGroup* g, hipStream_t s) {
-    long total = 0;
-    for (int i = 0; i < g->nprob; i++) total += mv_tiles_for(g->p[i].OC, g->p[i].nb * 32, MV_U);
+    auto tiles_at = [&](int U) {
+        long n = 0;
+        for (int i = 0; i < g->nprob; i++) n += mv_tiles_for(g->p[i].OC, g->p[i].nb * 32, U);
+        return n;
+    };
+    long total = tiles_at(MV_U);
     if (total <= 0) return 0;
-    const int U = total >= MV_WIDE_MIN_TILES ? MV_U_WIDE : MV_U;
+    const int U = total >= MV_WIDE_MIN_TILES ? MV_U_WIDE
+                  : tiles_at(1) <= MV_CUS    ? 1
+                  : tiles_at(2) <= MV_CUS    ? 2
+                                             : MV_U;
     total = 0;
     for (int i = 0; i < g->nprob; i++) {
         g->p[i].tiles = mv_tiles_for(g->p[i].OC, g->p[i].nb * 32, U);
@@ -663,10 +684,14 @@ static int launch_group(MvGroup* g, hipStream_t s) {
     const dim3 grid((unsigned)total), tb(MV_THREADS);
     if (QF == QF_Q4) {
         if (U == MV_U_WIDE) hipLaunchKernelGGL(k_q4_matvec<MV_U_WIDE>, grid, tb, 0, s, *g);
-        else hipLaunchKernelGGL(k_q4_matvec<MV_U>, grid, tb, 0, s, *g);
+        else if (U == MV_U) hipLaunchKernelGGL(k_q4_matvec<MV_U>, grid, tb, 0, s, *g);
+        else if (U == 2) hipLaunchKernelGGL(k_q4_matvec<2>, grid, tb, 0, s, *g);
+        else hipLaunchKernelGGL(k_q4_matvec<1>, grid, tb, 0, s, *g);
     } else {
         if (U == MV_U_WIDE) hipLaunchKernelGGL(k_q8_matvec<MV_U_WIDE>, grid, tb, 0, s, *g);
-        else hipLaunchKernelGGL(k_q8_matvec<MV_U>, grid, tb, 0, s, *g);
+        else if (U == MV_U) hipLaunchKernelGGL(k_q8_matvec<MV_U>, grid, tb, 0, s, *g);
+        else if (U == 2) hipLaunchKernelGGL(k_q8_matvec<2>, grid, tb, 0, s, *g);
+        else hipLaunchKernelGGL(k_q8_matvec<1>, grid, tb, 0, s, *g);
     }
     BMK_LAUNCH_CHECK();
     return 0;

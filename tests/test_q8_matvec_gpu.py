@@ -58,6 +58,34 @@ def test_matvec_integer_exact_bitwise(be):
     assert np.array_equal(y.astype(np.float64), r)
 
 
+@pytest.mark.parametrize("fmt", ["q8", "q4"])
+@pytest.mark.parametrize("C", [32, 288, 960, 4096])
+def test_matvec_rows_per_lane_bitwise(be, fmt, C):
+    """A row's sum does not depend on how many rows the launch has, so on the rows per lane that its size selects (one,
+    two, four, eight): the same bits for the same rows, against 64 bits once."""
+    slots = 256 // (C // 32)
+    sizes = [slots * 256 * 16, slots * 256 * 3, slots * 256 + 1, slots * 256, slots, 1]
+    OC = sizes[0]
+    pack, blk = {"q8": (po.quantize_q8, 36), "q4": (po.quantize_q4, 20)}[fmt]
+    base = bmhip.synth_normal(bmhip.synth_seed(9, 1, 0, C), 0.02, min(OC, 4096) * C)
+    w = np.tile(pack(base), -(-OC // 4096))[:OC * (C // 32) * blk]
+    x = bmhip.synth_normal(bmhip.synth_seed(9, 2, 0, C), 1.0, C)
+    bw, bx = be.upload(w), be.upload(x)
+    full = None
+    for n in sizes:
+        by = be.alloc(n * 4)
+        assert be.dispatch(f"matmul_forward_{fmt}_vec", [bx, bw, by, by, be.params(1, C, n, 0)], (n * 128, 1),
+                           (128,)) == 0
+        y = by.read(np.float32)
+        if full is None:
+            full = y
+        assert np.array_equal(y, full[:n]), n
+    n = min(OC, 4096)
+    f64 = po.q8_matvec_f64 if fmt == "q8" else po.q4_matvec_f64
+    r = f64(w[:n * (C // 32) * blk], x, 1, C, n)
+    assert normwise(full[:n], r) <= RTOL
+
+
 def test_matvec_bias(be):
     OC, C = 300, 576
     w = po.quantize_q8(bmhip.synth_normal(11, 0.02, OC * C))
