@@ -689,6 +689,32 @@ def test_persistent_step_small_shapes(dims, host_weights):
     b.close()
 
 
+@pytest.mark.parametrize("B", [1, 20], ids=["b1", "b20"])
+@pytest.mark.parametrize("dims", [
+    dict(D=416, H=2048, NH=6, NKV=3, HD=64, L=2, V=512),  # 13, 12 and 64 blocks per row: three batches of a row sum
+    dict(D=1024, H=768, NH=8, NKV=2, HD=64, L=2, V=512),  # 24: one whole batch; every lane of the norm
+    dict(D=800, H=832, NH=8, NKV=2, HD=64, L=2, V=512),   # 25 and 26: one block past a batch
+    dict(D=32, H=32, NH=1, NKV=1, HD=64, L=2, V=512),     # one block per row, one row per workgroup
+], ids=["h2048", "d1024", "d800", "d32"])
+def test_persistent_step_row_shapes(dims, B):
+    """Rows of 1 to 64 blocks in the persistent step against the per-phase kernels, one and two sequences an instance."""
+    a = bmhip.Engine(dims, max_seq_len=32, seed=17, batch=B)
+    b = bmhip.Engine(dims, max_seq_len=32, seed=17, batch=B)
+    try:
+        if not a.set_persistent(True):
+            pytest.skip("the persistent step kernel is not available on this device")
+        assert b.set_persistent(False)
+        for pos in range(12):
+            t = ((37 * pos + 11 + 5 * np.arange(B)) % dims["V"]).astype(np.int32)
+            ya, yb = (e.step(int(t[0])).reshape(1, -1) if B == 1 else e.step_batch(t) for e in (a, b))
+            for r in range(B):
+                assert normwise(ya[r], yb[r].astype(np.float64)) <= LOGIT_TOL, (pos, r)
+        assert a.persist_test_fault(0) == (1, 0)
+    finally:
+        a.close()
+        b.close()
+
+
 def test_persistent_step_long_context():
     """Positions past 640: each of the ten key chunks of an attention piece
     holds more than 64 keys, so a piece walks several sub-chunks (keys and
