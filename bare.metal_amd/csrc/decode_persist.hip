@@ -28,12 +28,11 @@
  *     merged attention output, the q/k/v of a KV head) issues all of its
  *     loads before it waits on any,
  *     an attention piece's cached keys and values first;
- *   - the weights of the next matvec phase are issued right after a
- *     phase's inputs have arrived (o in phase 1, the second RMSNorm in phase
- *     2, gate/up in phase 3 behind the merged output, down in phase 4, the
- *     next layer's q/k/v and
- *     first RMSNorm in phase 5), so they stream in while the phase computes,
- *     into registers of their own (per-phase pass counts P_QKV, P_O, P_GU,
+ *   - the weights of the next matvec phase are issued behind a phase's
+ *     products, pass by pass (o in phase 1, the second RMSNorm in phase 2,
+ *     gate/up in phase 3, down in phase 4, the next layer's q/k/v and first
+ *     RMSNorm in phase 5), so they stream in while the phase computes, into
+ *     registers of their own (per-phase pass counts P_QKV, P_O, P_GU,
  *     P_DN);
  *   - barriers inside a workgroup order LDS only (an LDS fence), so they
  *     do not wait for those weights;
@@ -51,8 +50,12 @@
  *     divisions and about 80 address instructions per phase before);
  *   - row sums read LDS six blocks at a time, P.V sixteen keys at a time,
  *     and lanes without an element of an exchanged vector load nothing.
- * SmolLM2-135M, GPU time of a step: 554 -> 518 us at batch 1, 866 -> 807 at
- * batch 32, the same bits.
+ *   - the merge of a share's partials takes a lane per (element, chunk)
+ *     (2.20 -> 1.06 us from a workgroup's partials to its share, and 1.25 ->
+ *     0.48 us more until the others' are in).
+ * SmolLM2-135M, GPU time of a step: 554 us without these, 518 without the
+ * last and with the next weights issued in front of the products, 451 now (batch
+ * 32: 866, 807, 748).
  *
  * Instances on one XCD each: MI355X hands workgroups to its 8 XCDs
  * round-robin (b to XCD (b + start) % 8, the start depending on the
@@ -153,7 +156,7 @@ __device__ __forceinline__ int tid() {
 
 static_assert(2 * KCH * HD <= KV_LDS, "a sub-chunk's keys and values fit their LDS");
 static_assert(4 * HD + 2 * HD <= PS_OFF && PS_OFF + (PT / 64) * KCH <= XS_MAX, "q, k, v and the probabilities share xs");
-static_assert(APR % 2 == 0, "partials load as 16-byte pairs of exchanged values");
+static_assert(DEC_PERSIST_NCH <= 16 && DEC_PERSIST_NCH_B <= 16, "the merge holds an element's chunks in 16 lanes");
 static_assert(P_QKV <= P_MAX && P_O <= P_MAX && P_GU <= P_MAX && P_DN <= P_MAX, "pass caps");
 
 /* Keeps the compiler from moving instructions across this point: loads
@@ -348,37 +351,46 @@ __device__ __forceinline__ void pin(Blk& b) {
     asm volatile("" : "+v"(b.q1.x), "+v"(b.q1.y), "+v"(b.q1.z), "+v"(b.q1.w));
 }
 
-/* Issues the share's block loads (one block per pass) into blk. */
+/* Issues part `part` of `parts` of a share's block loads (one block per pass) into blk. */
 template <int NP>
-__device__ __forceinline__ void mv_fetch(const unsigned char* wl, const unsigned int (&off)[NP], Blk (&blk)[NP]) {
+__device__ __forceinline__ void mv_fetch(const unsigned char* wl, const unsigned int (&off)[NP], Blk (&blk)[NP],
+                                         int part = 0, int parts = 1) {
 #pragma unroll
-    for (int p = 0; p < NP; p++) blk[p] = load_block(wl + off[p]);
+    for (int p = 0; p < NP; p++)
+        if (p * parts / NP == part) blk[p] = load_block(wl + off[p]);
 }
 
 /* The block products of the fetched blocks with each of the NB staged
  * vectors (vector j at xs + j * xs_len(C)) into red[j][local row][nb].
- * Returns whether the workgroup gives up (*bad as of the barrier before;
- * read beside the vectors, so that no wave waits for it alone). */
-template <int NB, int NP>
+ * issue(p) issues part p of NP of the next phase's loads behind pass p's
+ * products: the address unit takes about 20 cycles for each (64 lanes 36
+ * bytes apart), which held the whole phase up in front of them.  Returns
+ * whether the workgroup gives up (*bad as of the barrier before; read beside
+ * the vectors, so that no wave waits for it alone). */
+template <int NB, int NP, typename Issue>
 __device__ __forceinline__ bool mv_products(const MvShare& j, int n, Blk (&blk)[NP], const float* xs, int C, float* red,
-                                            const int* bad) {
-    const int t = tid(), tot = n * j.nb;
+                                            const int* bad, Issue&& issue) {
+    const int t = tid(), tot = t < j.sn ? n * j.nb : 0;
     const int stop = *bad;
-    if (t < j.sn) {
 #pragma unroll
-        for (int s = 0; s < NB; s++) {
-            const float* xb = xs + s * xs_len(C) + XB * j.bc;
-            float xv[32];
+    for (int s = 0; s < NB; s++) {
+        const float* xb = xs + s * xs_len(C) + XB * j.bc;
+        float xv[32];
 #pragma unroll
-            for (int i = 0; i < 32; i += 4) {
-                const float4 v = *(const float4*)&xb[i];
-                xv[i] = v.x; xv[i + 1] = v.y; xv[i + 2] = v.z; xv[i + 3] = v.w;
-            }
+        for (int i = 0; i < 32; i += 4) {
+            const float4 v = *(const float4*)&xb[i];
+            xv[i] = v.x; xv[i + 1] = v.y; xv[i + 2] = v.z; xv[i + 3] = v.w;
+        }
 #pragma unroll
-            for (int p = 0; p < NP; p++) {
-                const int e = t + p * j.sn;
-                if (s) pin(blk[p]); /* its codes converted again, not kept from the sequence before */
-                if (e < tot) red[s * tot + e] = block_dot(blk[p], xv);
+        for (int p = 0; p < NP; p++) {
+            const int e = t + p * j.sn;
+            if (s) pin(blk[p]); /* its codes converted again, not kept from the sequence before */
+            const float v = block_dot(blk[p], xv);
+            if (e < tot) red[s * n * j.nb + e] = v;
+            if (s == 0) {
+                issue_order();
+                issue(p);
+                issue_order();
             }
         }
     }
@@ -421,13 +433,14 @@ __device__ __forceinline__ void split_entry(int e, int n, int& s, int& o) {
  * residual y[r0 + o] = xres += sum (also stored to plain[s * ldy + r0 + o]
  * when plain is given).  The residual rows (s, o) a workgroup updates are
  * entries e = s * nout + o, entry e in xres[e / 64] of thread 4 (e % 64).
- * Returns mv_products' verdict, the outputs unwritten if it is to give up. */
-template <int NB, int NP>
+ * issue as for mv_products; returns its verdict, the outputs unwritten if the
+ * workgroup is to give up. */
+template <int NB, int NP, typename Issue>
 __device__ __forceinline__ bool mv_finish(const MvShare& j, Blk (&blk)[NP], const float* xs, int C, float* red,
                                           const int* bad, xv_t* y, int ldy, unsigned int ep, float (&xres)[NB],
-                                          float* plain) {
+                                          float* plain, Issue&& issue) {
     const int nb = j.nb, nout = j.r1 - j.r0, t = tid(), n = mv_rows(j), tot = NB * nout;
-    if (mv_products<NB>(j, n, blk, xs, C, red, bad)) return true;
+    if (mv_products<NB>(j, n, blk, xs, C, red, bad, issue)) return true;
     if (j.glu) {
         constexpr int EP = PT / 8; /* entries of a pass; two passes' chains side by side */
         for (int e0 = 0; e0 < tot; e0 += 2 * EP) {
@@ -728,48 +741,67 @@ __device__ __forceinline__ void attn_empty(const DecPersist& a, const Piece& p, 
 /* This workgroup's share of the attention output of the NB sequences
  * (elements [o0, o1) of NB x NH*HD, split evenly over the working
  * workgroups), merged from the partials of its nch chunks (exchanged with
- * epoch ep) by wave 0, one element per lane, and exchanged with epoch ep at
- * att: out = sum_c e^(m_c - M) acc_c / sum_c e^(m_c - M) l_c (chunks in
- * order; e^(m_c - M) = 0 for a chunk without keys).  Lanes past the share
- * load and store nothing. */
-template <int NB>
+ * epoch ep) and exchanged with epoch ep at att: out = sum_c e^(m_c - M) acc_c
+ * / sum_c e^(m_c - M) l_c (e^(m_c - M) = 0 for a chunk without keys).  One
+ * lane per (element, chunk), the chunks of an element in GL neighbouring
+ * lanes (nch <= GL): three loads and one exponential a lane, where one lane
+ * per element loaded 30 values and added ten chunks in turn.  R rounds hold
+ * the largest share (NB * 1024 elements over the workgroups). */
+template <int NB, int GL>
 __device__ __forceinline__ void attn_merge_share(const DecPersist& a, int nch, int w, const xv_t* apart, xv_t* att,
                                                  unsigned int ep, const Sync& sy) {
-    if (tid() >= 64) return;
-    constexpr int CM = DEC_PERSIST_NCH > DEC_PERSIST_NCH_B ? DEC_PERSIST_NCH : DEC_PERSIST_NCH_B;
-    const int tot = NB * a.QD;
+    constexpr int R = NB * QR * GL / DEC_PERSIST_WGS;
+    static_assert(R * (PT / GL) * DEC_PERSIST_WGS == NB * QR * PT, "the rounds cover the largest share");
+    const int tot = NB * a.QD, t = tid(), c = t % GL;
     const int o0 = (int)((long)tot * w / DEC_PERSIST_WGS), o1 = (int)((long)tot * (w + 1) / DEC_PERSIST_WGS);
-    const int i = o0 + tid();
-    int sq, e;
-    split_entry<NB>(i < o1 ? i : o0, a.QD, sq, e);
-    const int h = e / HD, d = e - h * HD;
-    const xv_t* pr = apart + (size_t)(sq * a.NH + h) * nch * APR;
-    auto addr = [&](int k) {
-        const int c = min(k / 3, nch - 1), f = k - 3 * (k / 3);
-        return pr + c * APR + (f == 2 ? 2 + d : f);
-    };
-    xv_t u[3 * CM];
+    const xv_t* pr[R];
+    int at[R];
+    bool has[R];
+    xv_t u[3 * R];
 #pragma unroll
-    for (int k = 0; k < 3 * CM; k++) {
-        u[k] = (xv_t)ep << 32;
-        if (i < o1) u[k] = get_xv(addr(k));
-    }
-    poll_xv<3 * CM>([&](int k) { return (unsigned int)(u[k] >> 32) == ep; }, [&](int k) { u[k] = get_xv(addr(k)); },
-                    sy);
-    float M = -INFINITY;
-#pragma unroll
-    for (int c = 0; c < CM; c++)
-        if (c < nch) M = fmaxf(M, xv_val(u[3 * c]));
-    float L = 0.f, A = 0.f;
-#pragma unroll
-    for (int c = 0; c < CM; c++)
-        if (c < nch) {
-            const float m = xv_val(u[3 * c]);
-            const float wc = m == -INFINITY ? 0.f : expf(m - M);
-            L = fmaf(wc, xv_val(u[3 * c + 1]), L);
-            A = fmaf(wc, xv_val(u[3 * c + 2]), A);
+    for (int r = 0; r < R; r++) {
+        const int i = o0 + t / GL + r * (PT / GL);
+        at[r] = i;
+        has[r] = i < o1 && c < nch;
+        int sq, e;
+        split_entry<NB>(min(i, tot - 1), a.QD, sq, e);
+        pr[r] = apart + ((size_t)(sq * a.NH + e / HD) * nch + min(c, nch - 1)) * APR;
+        u[3 * r] = ((xv_t)ep << 32) | __float_as_uint(-INFINITY);
+        u[3 * r + 1] = u[3 * r + 2] = (xv_t)ep << 32;
+        if (has[r]) {
+            u[3 * r] = get_xv(pr[r]);
+            u[3 * r + 1] = get_xv(pr[r] + 1);
+            u[3 * r + 2] = get_xv(pr[r] + 2 + e % HD);
         }
-    if (i < o1) put_xv(att + i, A / L, ep);
+    }
+    poll_xv<3 * R>([&](int k) { return (unsigned int)(u[k] >> 32) == ep; },
+                   [&](int k) {
+                       const int f = k % 3;
+                       u[k] = get_xv(pr[k / 3] + (f == 2 ? 2 + at[k / 3] % HD : f));
+                   },
+                   sy);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const float m = xv_val(u[3 * r]);
+        float M = m;
+        M = fmaxf(M, dpp<DPP_XOR1>(M));
+        M = fmaxf(M, dpp<DPP_XOR2>(M));
+        M = fmaxf(M, dpp<DPP_HALF_MIRROR>(M));
+        if (GL == 16) M = fmaxf(M, dpp<DPP_MIRROR>(M));
+        const float wc = m == -INFINITY ? 0.f : expf(m - M);
+        float L = wc * xv_val(u[3 * r + 1]), A = wc * xv_val(u[3 * r + 2]);
+        L += dpp<DPP_XOR1>(L);
+        A += dpp<DPP_XOR1>(A);
+        L += dpp<DPP_XOR2>(L);
+        A += dpp<DPP_XOR2>(A);
+        L += dpp<DPP_HALF_MIRROR>(L);
+        A += dpp<DPP_HALF_MIRROR>(A);
+        if (GL == 16) {
+            L += dpp<DPP_MIRROR>(L);
+            A += dpp<DPP_MIRROR>(A);
+        }
+        if (has[r] && c == 0) put_xv(att + at[r], A / L, ep);
+    }
 }
 
 /* HW_REG_XCC_ID bits [3:0] (s_getreg_b32 hwreg(HW_REG_XCC_ID, 0, 4)): the
@@ -888,9 +920,9 @@ __global__ __launch_bounds__(PT) void k_dec_persist(DecPersist a) {
         }, og);
         mv_offsets(sd, d1 - d0, w0, [&](int i) { return (unsigned int)a.off[6] + (d0 + i) * rowH; }, od);
     }
-    auto finish_qkv = [&](Blk(&blk)[P_QKV], unsigned int e) {
+    auto finish_qkv = [&](Blk(&blk)[P_QKV], unsigned int e, auto&& issue) {
         const int n = s1 - s0, tot = NB * n, t = tid();
-        if (mv_products<NB>(sq, n, blk, xs, D, red, &bad)) return true;
+        if (mv_products<NB>(sq, n, blk, xs, D, red, &bad, issue)) return true;
         for (int e0 = 0; e0 < tot; e0 += PT / 4) {
             const int ei = e0 + (t >> 2);
             int sb, r;
@@ -926,11 +958,9 @@ __global__ __launch_bounds__(PT) void k_dec_persist(DecPersist a) {
             } else {
                 get_vec<NB>(xf, D, ep(l - 1, 5), v, sy);
             }
-            issue_order();
-            mv_fetch(wl, oo, bo);
             norm_to_lds<NB>(v, D, nw, a.eps, xs, sh);
         }
-        if (finish_qkv(bq, ep(l, 1))) return;
+        if (finish_qkv(bq, ep(l, 1), [&](int p) { mv_fetch(wl, oo, bo, p, P_QKV); })) return;
         /* 2. RoPE + KV append + attention pieces.  The piece's cached keys and
          * values (positions before pos, written by earlier steps) do not
          * depend on this step's q, k, v: their loads go first. */
@@ -956,24 +986,25 @@ __global__ __launch_bounds__(PT) void k_dec_persist(DecPersist a) {
         }
         /* 3. merge (this workgroup's share) + o + residual; gate/up weights
          * stream in behind the merged output */
-        attn_merge_share<NB>(a, nch, w, apf, attf, ep(l, 2), sy);
+        if (NB == 2 && nch <= 8) attn_merge_share<NB, 8>(a, nch, w, apf, attf, ep(l, 2), sy);
+        else attn_merge_share<NB, 16>(a, nch, w, apf, attf, ep(l, 2), sy);
         {
             float v[NB][QR];
             get_vec<NB>(attf, QD, ep(l, 2), v, sy);
-            issue_order();
-            mv_fetch(wl, og, bg);
             vec_to_lds(v, QD, xs);
         }
-        if (mv_finish<NB>(so, bo, xs, QD, red, &bad, xf, D, ep(l, 3), xres, nullptr)) return;
+        if (mv_finish<NB>(so, bo, xs, QD, red, &bad, xf, D, ep(l, 3), xres, nullptr,
+                          [&](int p) { mv_fetch(wl, og, bg, p, P_O); }))
+            return;
         /* 4. RMSNorm + gate, up + SwiGLU; down's weights stream in behind x */
         {
             float v[NB][NW];
             get_vec<NB>(xf, D, ep(l, 3), v, sy);
-            issue_order();
-            mv_fetch(wl, od, bd);
             norm_to_lds<NB>(v, D, nw, a.eps, xs, sh);
         }
-        if (mv_finish<NB>(sg, bg, xs, D, red, &bad, hf, H, ep(l, 4), xres, nullptr)) return;
+        if (mv_finish<NB>(sg, bg, xs, D, red, &bad, hf, H, ep(l, 4), xres, nullptr,
+                          [&](int p) { mv_fetch(wl, od, bd, p, P_GU); }))
+            return;
         /* 5. down + residual; the next layer's q, k, v and first RMSNorm
          * weights stream in behind h (after the last layer: the last
          * layer's again, unused; no branch, so that h's loads stay first).
@@ -981,15 +1012,15 @@ __global__ __launch_bounds__(PT) void k_dec_persist(DecPersist a) {
         {
             float v[NB][XR];
             get_vec<NB>(hf, H, ep(l, 4), v, sy);
-            issue_order();
-            const int ln = min(l + 1, a.L - 1);
-            wl = a.w + (size_t)ln * a.layer_bytes;
-            mv_fetch(wl, oq, bq);
-            fetch_norm(a.ln1 + (size_t)ln * D, nw);
-            issue_order();
             vec_to_lds(v, H, xs);
         }
-        if (mv_finish<NB>(sd, bd, xs, H, red, &bad, xf, D, ep(l, 5), xres, l == a.L - 1 ? a.x + (size_t)b0 * D : nullptr))
+        const int ln = min(l + 1, a.L - 1);
+        wl = a.w + (size_t)ln * a.layer_bytes;
+        if (mv_finish<NB>(sd, bd, xs, H, red, &bad, xf, D, ep(l, 5), xres, l == a.L - 1 ? a.x + (size_t)b0 * D : nullptr,
+                          [&](int p) {
+                              mv_fetch(wl, oq, bq, p, P_DN);
+                              if (p == P_DN - 1) fetch_norm(a.ln1 + (size_t)ln * D, nw);
+                          }))
             return;
     }
 }
