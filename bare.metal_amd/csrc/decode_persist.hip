@@ -30,7 +30,7 @@
  *     an attention piece's cached keys and values first;
  *   - the weights of the next matvec phase are issued behind a phase's
  *     products, pass by pass (o in phase 1, the second RMSNorm in phase 2,
- *     gate/up in phase 3, down in phase 4, the next layer's q/k/v and first
+ *     gate/up in phases 2 and 3, down in phase 4, the next layer's q/k/v and first
  *     RMSNorm in phase 5), so they stream in while the phase computes, into
  *     registers of their own (per-phase pass counts P_QKV, P_O, P_GU,
  *     P_DN);
@@ -54,8 +54,8 @@
  *     (2.20 -> 1.06 us from a workgroup's partials to its share, and 1.25 ->
  *     0.48 us more until the others' are in).
  * SmolLM2-135M, GPU time of a step: 554 us without these, 518 without the
- * last and with the next weights issued in front of the products, 451 now (batch
- * 32: 866, 807, 748).
+ * last and with the next weights issued in front of the products, 431 now (batch
+ * 32: 866, 807, 723).
  *
  * Instances on one XCD each: MI355X hands workgroups to its 8 XCDs
  * round-robin (b to XCD (b + start) % 8, the start depending on the
@@ -113,6 +113,7 @@ constexpr int PT = 256;              /* threads per workgroup */
 constexpr int P_QKV = 4;             /* most row passes of a lane: q/k/v phase */
 constexpr int P_O = 2;               /*   o projection */
 constexpr int P_GU = 7;              /*   gate/up (two local rows per output) */
+
 constexpr int P_DN = 4;              /*   down projection */
 constexpr int P_MAX = 8;
 constexpr int XS_MAX = 4096;         /* floats of the staged input vector */
@@ -351,13 +352,13 @@ __device__ __forceinline__ void pin(Blk& b) {
     asm volatile("" : "+v"(b.q1.x), "+v"(b.q1.y), "+v"(b.q1.z), "+v"(b.q1.w));
 }
 
-/* Issues part `part` of `parts` of a share's block loads (one block per pass) into blk. */
-template <int NP>
+/* Issues part `part` of `parts` of a share's block loads of passes P0 .. P1 - 1 (one block per pass) into blk. */
+template <int NP, int P0 = 0, int P1 = NP>
 __device__ __forceinline__ void mv_fetch(const unsigned char* wl, const unsigned int (&off)[NP], Blk (&blk)[NP],
                                          int part = 0, int parts = 1) {
 #pragma unroll
-    for (int p = 0; p < NP; p++)
-        if (p * parts / NP == part) blk[p] = load_block(wl + off[p]);
+    for (int p = P0; p < P1; p++)
+        if ((p - P0) * parts / (P1 - P0) == part) blk[p] = load_block(wl + off[p]);
 }
 
 /* The block products of the fetched blocks with each of the NB staged
@@ -932,6 +933,12 @@ __global__ __launch_bounds__(PT) void k_dec_persist(DecPersist a) {
         }
         return false;
     };
+    /* Passes of gate/up whose weights are issued before the attention: gate
+     * and up are half of a layer's weights (2 MB at 135M, through one XCD's
+     * fabric port), and issued in phase 3 alone they arrived after phase 4
+     * wanted them.  0, 2, 3, 4, 5 passes: 452, 440, 438, 434, 438 us a step at
+     * batch 1; 751, 728, 723, 731, 731 at batch 32. */
+    constexpr int GE = NB == 1 ? 4 : 3;
     auto fetch_norm = [&](const float* nwp, float(&nw)[NW]) { load_vec(nwp, D, nw); };
 
     Blk bq[P_QKV], bo[P_O], bg[P_GU], bd[P_DN];
@@ -979,6 +986,7 @@ __global__ __launch_bounds__(PT) void k_dec_persist(DecPersist a) {
             }
             issue_order();
             fetch_norm(a.ln2 + (size_t)l * D, nw);
+            mv_fetch<P_GU, 0, GE>(wl, og, bg);
             lds_barrier();
             if (bad) return;
             if (live) attn_compute(a, pc, pos, rc, rs, ar, xs, big, apf, ep(l, 2));
@@ -994,7 +1002,7 @@ __global__ __launch_bounds__(PT) void k_dec_persist(DecPersist a) {
             vec_to_lds(v, QD, xs);
         }
         if (mv_finish<NB>(so, bo, xs, QD, red, &bad, xf, D, ep(l, 3), xres, nullptr,
-                          [&](int p) { mv_fetch(wl, og, bg, p, P_O); }))
+                          [&](int p) { mv_fetch<P_GU, GE, P_GU>(wl, og, bg, p, P_O); }))
             return;
         /* 4. RMSNorm + gate, up + SwiGLU; down's weights stream in behind x */
         {
