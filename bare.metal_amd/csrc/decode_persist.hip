@@ -82,8 +82,14 @@
  * through the chain of phases, on every workgroup's previous use of the
  * buffer (a workgroup writes x in phase 5 only after reading all of h, which
  * every workgroup wrote after reading x in phase 4, and so on; the
- * conditions are listed at dec_persist_ok and checked on the host).  The
- * spins are bounded in time: on timeout a workgroup sets
+ * conditions are listed at dec_persist_ok and checked on the host).  Waves
+ * of one workgroup go apart between its barriers in the same way, so an LDS
+ * word that one wave reads and another writes needs a barrier of the
+ * workgroup in between: the exchange orders a wave after the values that it
+ * loads itself, not after its siblings.  Each phase has one after it has
+ * staged its vectors and one after its block products; the attention, which
+ * ends without one, keeps what it reads last where phase 3 writes nothing
+ * (PLds::AT).  The spins are bounded in time: on timeout a workgroup sets
  * DecState.sync_error and leaves, and every other poll gives up once it
  * sees the flag, so the grid always drains.  A working workgroup that finds
  * itself on another XCD than a peer (HW_REG_XCC_ID, gathered per step in
@@ -126,7 +132,8 @@ constexpr int HD = 64;               /* head size */
 constexpr int KCH = 64;              /* keys of one attention sub-chunk (one per lane) */
 constexpr int KV_LDS = 2 * 64 * 64;  /* floats of one attention sub-chunk's keys and values in LDS */
 constexpr int APR = HD + 2;          /* one partial: max, sum, P.V[HD] */
-constexpr int PS_OFF = 1024;         /* attention: the waves' key probabilities in the staged-vector LDS, past q, k, v */
+constexpr int PS_OFF = 6 * HD;       /* attention: the waves' key probabilities, past q (at most four heads), k and v */
+constexpr int AT_LDS = PS_OFF + PT / 64 * KCH; /* floats of q, k, v and the probabilities */
 constexpr float SPIN_SECONDS = 0.2f;
 constexpr unsigned long long PEEK_TICKS = 1000; /* 10 us at 100 MHz: from then on a wait reads sync_error */
 /* LDS of an instance running NB sequences (NB = 1 or 2): the staged input
@@ -142,6 +149,11 @@ __device__ __forceinline__ int xs_len(int C) { return C / 32 * XB; }
 template <int NB>
 struct PLds {
     static constexpr int XS = NB == 1 ? XS_MAX : NB * (XS_SEQ / 32 * XB);
+    /* The attention's q, k, v and probabilities, past the attention output's
+     * staged vectors: no barrier lies between a slow wave's last reads of the
+     * one and a fast wave's writes of the other. */
+    static constexpr int AT = NB * (QR * PT / 32 * XB);
+    static_assert(AT + AT_LDS <= XS, "the attention output and q, k, v, probabilities lie side by side in xs");
     static constexpr int RED = P_MAX * PT * NB;
 };
 
@@ -156,7 +168,6 @@ __device__ __forceinline__ int tid() {
 }
 
 static_assert(2 * KCH * HD <= KV_LDS, "a sub-chunk's keys and values fit their LDS");
-static_assert(4 * HD + 2 * HD <= PS_OFF && PS_OFF + (PT / 64) * KCH <= XS_MAX, "q, k, v and the probabilities share xs");
 static_assert(DEC_PERSIST_NCH <= 16 && DEC_PERSIST_NCH_B <= 16, "the merge holds an element's chunks in 16 lanes");
 static_assert(P_QKV <= P_MAX && P_O <= P_MAX && P_GU <= P_MAX && P_DN <= P_MAX, "pass caps");
 
@@ -828,7 +839,7 @@ __global__ __launch_bounds__(PT) void k_dec_persist(DecPersist a) {
         if (threadIdx.x == 0) __hip_atomic_store(&a.st->sync_error, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return;
     }
-    __shared__ __attribute__((aligned(16))) float xs[PLds<NB>::XS]; /* staged input vectors, or the attention's q, k, v */
+    __shared__ __attribute__((aligned(16))) float xs[PLds<NB>::XS]; /* staged input vectors; the attention's q, k, v */
     __shared__ __attribute__((aligned(16))) float red[PLds<NB>::RED];
     __shared__ __attribute__((aligned(16))) float big[KV_LDS]; /* one attention sub-chunk's keys and values */
     __shared__ float sh[NB * (PT / 64)];
@@ -994,7 +1005,7 @@ __global__ __launch_bounds__(PT) void k_dec_persist(DecPersist a) {
             mv_fetch<P_GU, 0, GE>(wl, og, bg);
             lds_barrier();
             if (bad) return;
-            if (live) attn_compute(a, pc, pos, rc, rs, ar, xs, big, apf, ep(l, 2));
+            if (live) attn_compute(a, pc, pos, rc, rs, ar, xs + PLds<NB>::AT, big, apf, ep(l, 2));
             else if (has_piece) attn_empty(a, pc, apf, ep(l, 2));
         }
         /* 3. merge (this workgroup's share) + o + residual; gate/up weights
