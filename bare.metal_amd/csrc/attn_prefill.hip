@@ -32,10 +32,15 @@
  * 8 KB of LDS that only it uses.  The running maximum is moved only when a
  * score passes it by 2^8, so the reduction over the lane groups and the
  * rescaling of O are rare; sums stay far inside fp32's range and their
- * relative error is the same.
+ * relative error is the same.  A wave's two sub-blocks of a turn are summed
+ * on their own before they join O: with four waves the products straight into
+ * O are chains twice as long as with eight, and the error against 64 bits grew
+ * with the prompt (N(0, 1), 512 / 2048 / 4096 positions, 1e-7: eight waves 1.48 /
+ * 1.83 / 2.15, four 1.56 / 2.11 / 2.60, so 1.45 / 1.61 / 1.70).
  * GPU time per launch, back to back, before / now, 15 heads on 5 KV heads: 16
  * positions 6.1 / 4.4 us, 333 14.1 / 10.0, 512 21.9 / 14.0, 1024 61.2 / 32.7, 2048 198 / 92
- * (the products alone take 52); 9 heads on 3, 512 positions: 15.8 / 11.6.  8 waves
+ * (the products alone take 52); 9 heads on 3, 512 positions: 15.8 / 11.6; the
+ * turns' own sums cost 0.5-3% of that (2048: 98.35 -> 98.43, kernel trace).  8 waves
  * per workgroup: 104 us at 2048, 5.8 at 16; one sub-block at a time: the same
  * within 2%; a register budget for 4 waves per SIMD spills (193 us).
  */
@@ -128,8 +133,11 @@ __global__ __launch_bounds__(64 * AW) __attribute__((amdgpu_waves_per_eu(3, 3)))
     fetch_v(wave + AW, v1r);
     __builtin_amdgcn_sched_barrier(0);
     f32x4 acc[4]; /* O^T tile d: dims 16d + 4*grp + v, query col */
+    auto zero = [](f32x4* o) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int d = 0; d < 4; d++) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    };
+    zero(acc);
     float m = -INFINITY, l = 0.0f; /* m: per query (same in the 4 lane groups); l: this lane's keys */
 
     /* S^T[key 4*grp + v][query col] of a sub-block, times scale * log2(e) */
@@ -179,15 +187,19 @@ __global__ __launch_bounds__(64 * AW) __attribute__((amdgpu_waves_per_eu(3, 3)))
         f32x4 pv;
 #pragma unroll
         for (int v = 0; v < 4; v++) pv[v] = m > -INFINITY ? __builtin_amdgcn_exp2f(sv[v] - m) : 0.0f;
-        l += (pv.x + pv.y) + (pv.z + pv.w);
         return pv;
     };
+    auto sum4 = [](const f32x4& v) { return (v.x + v.y) + (v.z + v.w); };
     /* O^T[dim 16d + col'][query] += V^T[dim][key 4*grp + i] * P^T[key][query] */
-    auto values = [&](const float* v, const f32x4& pv) {
+    auto values = [&](const float* v, const f32x4& pv, f32x4* o) {
 #pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
-            for (int d = 0; d < 4; d++) acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[4 * i + d], pv[i], acc[d], 0, 0, 0);
+            for (int d = 0; d < 4; d++) o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[4 * i + d], pv[i], o[d], 0, 0, 0);
+    };
+    auto add = [&](const f32x4* o) {
+#pragma unroll
+        for (int d = 0; d < 4; d++) acc[d] += o[d];
     };
     float* Kw = &Ws[wave * 2 * 16 * HD];
     /* Below the diagonal two sub-blocks at a time, so that one's products run
@@ -203,10 +215,14 @@ __global__ __launch_bounds__(64 * AW) __attribute__((amdgpu_waves_per_eu(3, 3)))
         fetch_k(sb + 3 * AW, k1r);
         __builtin_amdgcn_sched_barrier(0);
         move_max(fmaxf(max4(sa), max4(sc)));
+        f32x4 o2[4]; /* a turn's own sum first: acc's chain has one rounding per 32 keys of the wave instead of eight */
+        zero(o2);
         const f32x4 pa = weights(sa);
-        values(v0r, pa);
+        values(v0r, pa, o2);
         const f32x4 pc = weights(sc);
-        values(v1r, pc);
+        values(v1r, pc, o2);
+        l += sum4(pa) + sum4(pc);
+        add(o2);
         __builtin_amdgcn_sched_barrier(0);
         fetch_v(sb + 2 * AW, v0r);
         fetch_v(sb + 3 * AW, v1r);
@@ -224,7 +240,12 @@ __global__ __launch_bounds__(64 * AW) __attribute__((amdgpu_waves_per_eu(3, 3)))
             for (int d = 0; d < 4; d++) vz[4 * i + d] = key < n ? v[4 * i + d] : 0.0f; /* past n there is nothing */
         }
         move_max(max4(sv));
-        values(vz, weights(sv));
+        f32x4 o2[4];
+        zero(o2);
+        const f32x4 pv = weights(sv);
+        l += sum4(pv);
+        values(vz, pv, o2);
+        add(o2);
     };
     if (sb < nsb) last_one(sb, k0r, v0r);
     if (sb + AW < nsb) last_one(sb + AW, k1r, v1r);
