@@ -40,7 +40,7 @@
  * GPU time per launch, back to back, before / now, 15 heads on 5 KV heads: 16
  * positions 6.1 / 4.4 us, 333 14.1 / 10.0, 512 21.9 / 14.0, 1024 61.2 / 32.7, 2048 198 / 92
  * (the products alone take 52); 9 heads on 3, 512 positions: 15.8 / 11.6; the
- * turns' own sums cost 0.5-3% of that (2048: 98.35 -> 98.43, kernel trace).  8 waves
+ * turns' own sums cost up to 4% of that (2048: 98.35 -> 98.43, kernel trace).  8 waves
  * per workgroup: 104 us at 2048, 5.8 at 16; one sub-block at a time: the same
  * within 2%; a register budget for 4 waves per SIMD spills (193 us).
  */
