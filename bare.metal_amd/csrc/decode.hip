@@ -1967,7 +1967,7 @@ static int launch_matmul_rows(const bmk_launch_t* a, int wf) {
     BMK_NEED_BYTES(a, 1, (size_t)OC * C * esz, "weight");
     if (hb) BMK_NEED_BYTES(a, 2, (size_t)OC * 4, "bias");
     BMK_NEED_BYTES(a, 3, (size_t)BT * OC * 4, "out");
-    if (rows_gemm_ok(BT, C, OC) && (((uintptr_t)a->dev[0] | (uintptr_t)a->dev[1]) & 3) == 0)
+    if (rows_gemm_ok(BT, C, OC, wf) && (((uintptr_t)a->dev[0] | (uintptr_t)a->dev[1]) & 3) == 0)
         return rows_gemm_launch((const float*)a->dev[0], (const void*)a->dev[1], wf, hb ? (const float*)a->dev[2] : nullptr,
                                 (float*)a->dev[3], BT, C, OC, a->stream);
     if (!head_shape_ok(C, wf)) {

@@ -13,7 +13,7 @@ enum { RG_F32 = 0, RG_BF16 = 2, RG_F16 = 3 }; /* weight formats, as the LM head'
 extern "C" {
 #endif
 /* whether rows_gemm_launch serves the shape */
-int rows_gemm_ok(int BT, int C, int OC);
+int rows_gemm_ok(int BT, int C, int OC, int wf);
 /* out[BT][OC] = x[BT][C] x w^T (+ bias); operands 4-byte aligned (16-bit weights 2-byte) */
 int rows_gemm_launch(const float* x, const void* w, int wf, const float* bias, float* out, int BT, int C, int OC,
                      hipStream_t s);

@@ -13,7 +13,9 @@
  * (conflict-free: rows are padded by four floats).
  * Two tile shapes (rg_launch):
  *   32 x 32, the four waves taking a quarter of each 128-wide K step, summed
- *   in LDS at the end: the most workgroups, for launches that fit one per CU;
+ *   in LDS at the end: the most workgroups, for launches that fit one per CU,
+ *   and for up to 32 rows, which a 64-row tile would leave half empty (8 x 960 ->
+ *   49152 68.5 / 41.3 us, 16 x 2560 -> 8192 no different);
  *   64 x 32, two waves along the rows and two along K: a third less operand
  *   traffic per product where the CUs would take several workgroups each.
  * Measured, C = 960, bf16 rows, 32 x 32 / 64 x 32 (us, back to back, one
@@ -39,7 +41,7 @@ constexpr int RG_NT = 256;
  * LM-head kernel's sums (normwise, C 960 / 2560: 1.2e-7 / 1.7e-7; with one
  * partial sum 2.8e-7, with four 1.5e-7 / 2.4e-7; eight cost 0.4 us). */
 constexpr int ACC = 8, FOLD = 8;
-/* a launch with more 32 x 32 tiles than this (one per CU) takes 64 x 32 ones */
+/* a launch of more rows than a tile's and more 32 x 32 tiles than this (one per CU) takes 64 x 32 ones */
 constexpr long RG_CU_TILES = 256;
 
 struct RgArgs {
@@ -204,7 +206,7 @@ __global__ __launch_bounds__(RG_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
 template <int WF>
 void rg_launch(const RgArgs& a, hipStream_t s) {
     const unsigned tn = (a.OC + 31) / 32;
-    if ((long)((a.BT + 31) / 32) * tn > RG_CU_TILES)
+    if (a.BT > 32 && (long)((a.BT + 31) / 32) * tn > RG_CU_TILES)
         hipLaunchKernelGGL((k_rows_gemm<WF, 2, 2>), dim3((a.BT + 63) / 64, tn), dim3(RG_NT), 0, s, a);
     else
         hipLaunchKernelGGL((k_rows_gemm<WF, 1, 4>), dim3((a.BT + 31) / 32, tn), dim3(RG_NT), 0, s, a);
@@ -212,13 +214,27 @@ void rg_launch(const RgArgs& a, hipStream_t s) {
 
 } // namespace
 
-/* Two rows over a long C stay with the LM-head kernel, whose workgroups take
- * three output rows each there: 2 x 2560 -> 960 13.5 us against 18.7 here, 2 x 1536
- * -> 576 11.5 / 12.2, but 2 x 960 -> 2560 9.7 / 9.1 and 2 x 576 -> 1536 9.0 / 6.7;
- * from three rows on this one is as fast or faster (3 x 2560 -> 960 18.4 / 18.6,
- * 3 x 960 -> 2560 12.6 / 9.1, 6 x 2560 -> 960 32.6 / 18.6). */
-extern "C" int rows_gemm_ok(int BT, int C, int OC) {
-    return (BT >= 3 || (BT == 2 && C <= 1024)) && C % 32 == 0 && OC <= 65535L * 32;
+/* A few rows stay with the LM-head kernel, which reads its weights once and
+ * applies them to each row in turn, where that takes less than a 32-row tile.
+ * Its cost grows with the rows and little with OC while the CUs last; here it is
+ * the chain over C, and past one tile per CU the tiles' count.  Both sides in
+ * us (head kernel / this one, kernel trace, bf16 rows):
+ *   up to one tile per CU   C = 960        1536         2560         4096         8192
+ *     2 rows                9.3 / 8.5      11.2 / 12.2  13.3 / 18.6  17.0 / 27.6  26.4 / 53.8
+ *     3 rows                12.2 / 8.8     15.3 / 12.0  18.2 / 18.6  23.6 / 27.6  37.1 / 53.2
+ *     4 rows                15.4 / 8.5     19.0 / 12.0  23.0 / 18.6  30.3 / 27.6  47.9 / 53.2
+ *     5 rows                18.3 / 8.9     22.8 / 12.2  27.8 / 18.5  37.1 / 27.6  59.3 / 53.4
+ *   more                    960 -> 16384   960 -> 49152 2048 -> 32000  4096 -> 16384
+ *     2 rows                10.3 / 15.8    34.3 / 44.1  60.4 / 55.8    76.0 / 55.2
+ *     3 rows                13.0 / 15.6    42.8 / 43.7  79.2 / 55.0    102.8 / 54.5
+ *     4 rows                16.2 / 15.6    51.7 / 43.0  98.2 / 54.3    129.5 / 54.5
+ * fp32 rows differ at three: 2560 -> 960 23.5 / 20.2, 4096 -> 40 34.1 / 29.8, 960 -> 49152 42.2 / 45.6, 8192 -> 2048
+ * 34.6 / 59.0 (five rows 57.8 / 59.5). */
+extern "C" int rows_gemm_ok(int BT, int C, int OC, int wf) {
+    if (BT < 2 || C % 32 != 0 || OC > 65535L * 32) return 0;
+    if ((OC + 31) / 32 > RG_CU_TILES) return BT >= 4 || C >= 2048;
+    const int most = BT == 2 ? 1024 : BT == 3 ? (wf == RG_F32 ? 4096 : 2560) : BT == 4 ? 4096 : C;
+    return C <= most;
 }
 
 extern "C" int rows_gemm_launch(const float* x, const void* w, int wf, const float* bias, float* out, int BT, int C,

@@ -530,6 +530,14 @@ def test_matmul_forward_rows(be, name, BT, C, OC, bias, off):
     assert (got[BT * OC:] == 7.0).all()
 
 
+@pytest.mark.parametrize("BT,C,OC", [(4, 64, 8225), (5, 96, 8225), (32, 64, 8193), (33, 64, 8193), (3, 64, 8193),
+                                     (2, 2080, 8193)])
+def test_matmul_forward_rows_many_outputs(be, BT, C, OC):
+    """More output tiles than CUs: up to 32 rows on 32-row tiles, 33 on 64-row ones, 3 short rows on the LM-head
+    kernel, 2 long ones not."""
+    test_matmul_forward_rows(be, "matmul_forward_bf16_simd", BT, C, OC, 1, 4)
+
+
 def test_matmul_forward_rows_nonfinite(be):
     """An infinite or NaN operand reaches its own row and column only, as in the plain sum."""
     BT, C, OC = 40, 256, 70

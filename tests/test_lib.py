@@ -52,6 +52,17 @@ def test_backend_abi_is_complete():
         assert hasattr(lib, n), n
 
 
+@pytest.mark.parametrize("BT,C,OC,bf16,f32", [
+    (1, 960, 960, 0, 0), (2, 1024, 960, 1, 1), (2, 1056, 960, 0, 0), (3, 2560, 960, 1, 1), (3, 4096, 4096, 0, 1),
+    (4, 4096, 40, 1, 1), (4, 8192, 2048, 0, 0), (5, 8192, 2048, 1, 1), (2, 576, 8192, 1, 1), (2, 576, 49152, 0, 0),
+    (3, 960, 49152, 0, 0), (4, 960, 49152, 1, 1), (2, 4096, 16384, 1, 1), (64, 30, 960, 0, 0),
+])
+def test_unquantized_matmul_of_a_few_rows_keeps_the_head_kernel(BT, C, OC, bf16, f32):
+    """Which shapes of the unquantized matmul names go to the tiled kernel: a few rows over an LM head's outputs or over
+    a long sum take up to 2.3 times as long there (both sides measured, rows_gemm.hip)."""
+    assert [bmhip.lib().rows_gemm_ok(BT, C, OC, wf) for wf in (2, 3, 0)] == [bf16, bf16, f32]
+
+
 def test_null_handles_are_safe():
     """*_free/destroy(NULL) are no-ops and NULL encoders/kernels are rejected
     (reference device.m:144-159,182-191; dispatch.m:56,110)."""
