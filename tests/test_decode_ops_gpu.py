@@ -220,6 +220,15 @@ def test_attention_forward_splits(be, NH, kv_mul, HD, S):
     assert nw(out.read(np.float32), want) <= TOL
 
 
+@pytest.mark.parametrize("NH,kv_mul,HD,S", [(8, 4, 32, 512), (8, 4, 32, 513), (7, 3, 64, 256), (7, 3, 64, 257),
+                                            (6, 6, 128, 256), (6, 6, 128, 257), (5, 2, 256, 128), (5, 2, 256, 129),
+                                            (9, 8, 16, 1024), (9, 8, 16, 1025), (3, 1, 64, 128)])
+def test_attention_forward_one_split(be, NH, kv_mul, HD, S):
+    """The last key count of one split (four tiles where a KV head has several query heads, else two; a workgroup per
+    query head) and the first of several."""
+    test_attention_forward_splits(be, NH, kv_mul, HD, S)
+
+
 def test_attention_forward_masked_and_nonfinite(be):
     """Scores of -inf drop their keys (here all but one key of one split), scores that are all -inf, +inf or NaN give
     NaN, as the unsplit softmax has them."""
