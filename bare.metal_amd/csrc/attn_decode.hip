@@ -8,15 +8,15 @@
  * SmolLM2-360M and 2048 keys, 1 us of HBM time, so one workgroup per query
  * head (15 workgroups walking all keys in turn) is a latency chain on a
  * nearly idle chip.  Here a workgroup takes one split of the keys of one KV
- * head and, past a few tiles of keys, serves up to four of its query heads, so
+ * head and, past two tiles of keys, serves up to four of its query heads, so
  * every K and V row is read once per four heads, and all of a tile's loads
  * are issued before the first is used.  The last workgroup of a KV head to
  * finish merges the splits' (max, sum, partial output) records.
  *
  * GPU time per launch, back to back, 15 query heads on 5 KV heads of 64, one
  * workgroup per head before / splits now: 301 keys 17.4 (9 heads on 3) / 6.6 us,
- * 2048 keys 155 / 7.5 us, 4096 keys 10.3 us; one key takes 3.2 us, four
- * tiles 5.2 us (kernel trace).  What is left is latency: loads, two handovers, the merge.  With 8
+ * 2048 keys 155 / 7.5 us, 4096 keys 10.3 us; one key takes 3.2 us, two
+ * tiles 3.9 us (kernel trace).  What is left is latency: loads, two handovers, the merge.  With 8
  * waves of 16 keys instead of 4: 0.2-0.9 us more up to 2048 keys, 1.6 us less
  * at 4096.  The merge reads at most 16 records of an output at once: 32
  * measured 0.3 us slower up to 1000 keys, and reading a clamped record again
@@ -268,26 +268,25 @@ __global__ __launch_bounds__(AT_NT) void k_attn_decode(AtArgs a) {
     }
 }
 
-/* Few keys take one split (no records, no merge) and one query head per
- * workgroup: up to four tiles where a split's workgroups would serve several
- * heads, whose scores one after another cost more than what they share of the
- * rows, else two.  us by kernel trace, workgroup per head before the splits /
- * splits of shared heads past two tiles / now, per head size and kv_mul: 64, 3:
- * 16 keys 5.0 / 4.3 / 3.2, 128 7.4 / 5.9 / 3.9, 256 11.6 / 6.6 / 5.2; 128, 4: 65 8.9 / 10.2 /
- * 5.4, 256 20.4 / 10.6 / 8.4; 32, 4: 1 4.1 / 5.0 / 3.3; 16, 4: 48 4.1 / 4.6 / 3.3; 256, 4: 48
- * 13.4 / 15.0 / 5.7, 128 22.0 / 13.3 / 8.8.  Five tiles: splits 6.0 us, one 5.7 (64,
- * 3), six: 6.0, 6.2; heads of their own, 256 and 128 keys (four tiles): splits 6.8
- * us, one 9.6. */
-constexpr int AT_ONE_TILES = 2, AT_ONE_TILES_SHARED = 4;
+/* Up to two tiles of keys take one split (no records, no merge) and one query
+ * head per workgroup: the scores of several heads one after another cost more
+ * than what they share of so few rows.  us by kernel trace, workgroup per head
+ * before the splits / shared heads / now, per head size and kv_mul: 64, 3: 16 keys
+ * 5.0 / 4.3 / 3.2, 128 7.4 / 5.9 / 3.9; 128, 4: 65 8.9 / 10.2 / 5.4; 32, 4: 1 4.1 / 5.0 / 3.3;
+ * 16, 4: 48 4.1 / 4.6 / 3.3; 256, 4: 48 13.4 / 15.0 / 5.7.  Three or four tiles of shared
+ * heads in one split are faster too (64, 3, 256 keys 6.6 / 5.2), but the sums of a
+ * workgroup get longer (error against 64 bits 1.41e-7 / 1.51e-7; 128, 4: 1.56e-7 /
+ * 1.80e-7). */
+constexpr int AT_ONE_TILES = 2;
 
-/* Keys per split (*keys, whole tiles) and splits: one for up to `one` tiles,
- * else as many splits as there are tiles, up to AT_MAX_SPLIT and what the
- * scratch memory holds. */
+/* Keys per split (*keys, whole tiles) and splits: one (AT_ONE_TILES), else as
+ * many splits as there are tiles, up to AT_MAX_SPLIT and what the scratch
+ * memory holds. */
 template <int HD>
-int at_split(int S, int one, int groups, int qh, size_t scratch_bytes, int* keys) {
+int at_split(int S, int groups, int qh, size_t scratch_bytes, int* keys) {
     const int tile = AtTile<HD>::KEYS, tiles = (S + tile - 1) / tile;
     size_t most = 1;
-    if (tiles > one && groups <= AT_MAX_GROUPS && scratch_bytes > AT_DONE_BYTES)
+    if (tiles > AT_ONE_TILES && groups <= AT_MAX_GROUPS && scratch_bytes > AT_DONE_BYTES)
         most = (scratch_bytes - AT_DONE_BYTES) / ((size_t)groups * qh * (HD + 2) * 4);
     most = std::min<size_t>(std::max<size_t>(most, 1), AT_MAX_SPLIT);
     const int per = (tiles + (int)most - 1) / (int)most;
@@ -297,13 +296,12 @@ int at_split(int S, int one, int groups, int qh, size_t scratch_bytes, int* keys
 
 template <int HD>
 int at_launch(AtArgs a, int groups, int qh, const bmk_launch_t* l) {
-    const int one = qh > 1 ? AT_ONE_TILES_SHARED : AT_ONE_TILES;
-    if (a.S <= one * AtTile<HD>::KEYS) { /* one head per workgroup */
+    if (a.S <= AT_ONE_TILES * AtTile<HD>::KEYS) { /* one head per workgroup */
         qh = 1;
         a.ng = a.kv_mul;
         groups = a.NH;
     }
-    a.nsplit = at_split<HD>(a.S, one, groups, qh, l->scratch_bytes, &a.keys);
+    a.nsplit = at_split<HD>(a.S, groups, qh, l->scratch_bytes, &a.keys);
     a.done = (unsigned int*)l->scratch;
     a.rec = a.nsplit > 1 ? (float*)((char*)l->scratch + AT_DONE_BYTES) : nullptr;
     const dim3 grid((unsigned)groups * a.nsplit), tb(AT_NT);
