@@ -120,8 +120,16 @@ __device__ __forceinline__ bf16x8 dq(const u32x4* q, int u, float s) {
     return __builtin_bit_cast(bf16x8, r);
 }
 
+/* Waves per SIMD that the compiler must leave room for.  With three steps in
+ * registers the Q4_0 64 x 64 forms came out at 260, one workgroup per CU, and
+ * gate/up of long prompts took longer (360M, 512 / 2000 tokens 19.4 / 49.8 us with
+ * two, 23.8 / 72.0 with one, 17.7 / 48.2 now). */
+constexpr int pfg_waves(int qf, int epi, int mi, int nj) {
+    return qf == QF_Q4 && mi == 2 && nj == 2 && epi != PFG_RESID ? 2 : 1;
+}
+
 template <int QF, int EPI, int MI, int NJ>
-__global__ __launch_bounds__(PNTH) void k_pf_gemm(PfgArgs a) {
+__global__ __launch_bounds__(PNTH, pfg_waves(QF, EPI, MI, NJ)) void k_pf_gemm(PfgArgs a) {
     constexpr int PTM = 32 * MI;  /* tile rows */
     constexpr int TW = 32 * NJ;   /* tile columns */
     constexpr int CPT = 8 * NJ;   /* epilogue columns per thread */
@@ -244,6 +252,8 @@ __global__ __launch_bounds__(PNTH) void k_pf_gemm(PfgArgs a) {
         }
 #pragma unroll
         for (int u = 0; u < 4; u++) {
+            /* all four fragments converted ahead of their products spill at 256 registers */
+            if (pfg_waves(QF, EPI, MI, NJ) == 2 && u == 2) __builtin_amdgcn_sched_barrier(0);
             bf16x8 fb[NJ], fa[MI];
 #pragma unroll
             for (int j = 0; j < NJ; j++) fb[j] = dq<QF>(st.q[j], u, st.s[j]);
