@@ -2202,11 +2202,13 @@ extern "C" int dec_pf_embed(const int* tok, const float* emb, float* x, int n, i
 /* RoPE + cache append of every position (unless the q/k/v GEMM's epilogue
  * did it, q's RoPE too: kv_done), then causal attention; the result goes to
  * out16 as bf16 in fragment order (the o-projection's operand).  Head size
- * 64: blocks of PQB positions per workgroup, written as bf16 directly; other
- * head sizes: one workgroup per (head, position) into a->out (fp32), then
- * the fragment-order cast (which also zeroes the columns past NH * HD). */
+ * 64, which needs kv_done (its kernel takes q as it is): ap_launch, written as
+ * bf16 directly; other head sizes: one workgroup per (head, position), which
+ * rotates q, into a->out (fp32), then the fragment-order cast (which also
+ * zeroes the columns past NH * HD). */
 extern "C" int dec_pf_attention(const DecAttn* a, const float* q, const float* k, const float* v, int n,
                                 unsigned short* out16, int kv_done, hipStream_t s) {
+    BMK_REQUIRE(a->HD != 64 || kv_done, "prefill attention: head size 64 takes q already rotated");
     if (!kv_done) {
         hipLaunchKernelGGL(k_pf_kv, dim3(n), dim3(NT), 0, s, *a, k, v);
         BMK_LAUNCH_CHECK();

@@ -63,6 +63,20 @@ def test_unquantized_matmul_of_a_few_rows_keeps_the_head_kernel(BT, C, OC, bf16,
     assert [bmhip.lib().rows_gemm_ok(BT, C, OC, wf) for wf in (2, 3, 0)] == [bf16, bf16, f32]
 
 
+def test_prefill_attention_of_head_size_64_needs_rotated_q(capfd):
+    """dec_pf_attention's kernel for head size 64 takes q as it is: a call that says q is not yet rotated (kv_done 0) is
+    refused before any launch.  Of DecAttn (decode_state.h) only HD is read ahead of that."""
+    class DecAttn(ctypes.Structure):
+        _fields_ = [("ptr", ctypes.c_void_p * 6), ("inv_freq", ctypes.c_float * 128), ("scale", ctypes.c_float),
+                    ("NH", ctypes.c_int), ("NKV", ctypes.c_int), ("HD", ctypes.c_int), ("KV", ctypes.c_int),
+                    ("MS", ctypes.c_int), ("L", ctypes.c_int), ("layer", ctypes.c_int)]
+
+    a = DecAttn(NH=3, NKV=1, HD=64, KV=64, MS=16, L=1)
+    none = ctypes.c_void_p(None)
+    assert bmhip.lib().dec_pf_attention(ctypes.byref(a), none, none, none, 4, none, 0, none) == -1
+    assert "takes q already rotated" in capfd.readouterr().err
+
+
 def test_null_handles_are_safe():
     """*_free/destroy(NULL) are no-ops and NULL encoders/kernels are rejected
     (reference device.m:144-159,182-191; dispatch.m:56,110)."""
