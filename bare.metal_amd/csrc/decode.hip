@@ -332,6 +332,7 @@ __device__ __forceinline__ unsigned long long* head_key(const DecHead& a, int b)
 /* Weight formats of the LM head rows: fp32, Q8_0 blocks, and two 16-bit
  * formats (bf16, IEEE fp16), each widened exactly to fp32. */
 enum { HW_F32 = 0, HW_Q8 = 1, HW_BF16 = 2, HW_F16 = 3 };
+static_assert((int)HW_F32 == RG_F32 && (int)HW_BF16 == RG_BF16 && (int)HW_F16 == RG_F16, "rows_gemm.h's formats");
 
 template <int WF>
 __device__ __forceinline__ int head_lanes(int D) { return WF == HW_F32 ? D / 16 : D / 32; }

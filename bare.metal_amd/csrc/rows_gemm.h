@@ -12,9 +12,9 @@ enum { RG_F32 = 0, RG_BF16 = 2, RG_F16 = 3 }; /* weight formats, as the LM head'
 #ifdef __cplusplus
 extern "C" {
 #endif
-/* whether rows_gemm_launch serves the shape */
+/* whether the shape (weights in format wf) is better served by rows_gemm_launch */
 int rows_gemm_ok(int BT, int C, int OC, int wf);
-/* out[BT][OC] = x[BT][C] x w^T (+ bias); operands 4-byte aligned (16-bit weights 2-byte) */
+/* out[BT][OC] = x[BT][C] x w^T (+ bias); x and w 4-byte aligned, C a multiple of 32; -1: refused */
 int rows_gemm_launch(const float* x, const void* w, int wf, const float* bias, float* out, int BT, int C, int OC,
                      hipStream_t s);
 #ifdef __cplusplus

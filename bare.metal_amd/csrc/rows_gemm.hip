@@ -239,6 +239,9 @@ extern "C" int rows_gemm_ok(int BT, int C, int OC, int wf) {
 
 extern "C" int rows_gemm_launch(const float* x, const void* w, int wf, const float* bias, float* out, int BT, int C,
                                 int OC, hipStream_t s) {
+    /* the loaders take 16 bytes from 4-byte aligned addresses, 16-bit weights too */
+    BMK_REQUIRE(BT > 0 && OC > 0 && C > 0 && C % 32 == 0 && OC <= 65535L * 32, "rows gemm: %d x %d -> %d", BT, C, OC);
+    BMK_REQUIRE((((uintptr_t)x | (uintptr_t)w) & 3) == 0, "rows gemm: operands must be 4-byte aligned");
     const RgArgs a = {x, w, bias, out, BT, C, OC};
     if (wf == RG_F32) rg_launch<RG_F32>(a, s);
     else if (wf == RG_BF16) rg_launch<RG_BF16>(a, s);

@@ -63,6 +63,15 @@ def test_unquantized_matmul_of_a_few_rows_keeps_the_head_kernel(BT, C, OC, bf16,
     assert [bmhip.lib().rows_gemm_ok(BT, C, OC, wf) for wf in (2, 3, 0)] == [bf16, bf16, f32]
 
 
+def test_unquantized_matmul_kernel_refuses_what_its_loads_cannot_take(capfd):
+    """Weights or inputs off a 4-byte boundary (16-bit weights too) and sums that are not whole 32-column blocks are
+    refused before any launch."""
+    p = ctypes.c_void_p
+    for x, w, C in ((16, 18, 64), (18, 16, 64), (16, 16, 48)):
+        assert bmhip.lib().rows_gemm_launch(p(x), p(w), 2, p(None), p(16), 4, C, 32, p(None)) == -1
+        assert "rows gemm" in capfd.readouterr().err
+
+
 def test_prefill_attention_of_head_size_64_needs_rotated_q(capfd):
     """dec_pf_attention's kernel for head size 64 takes q as it is: a call that says q is not yet rotated (kv_done 0) is
     refused before any launch.  Of DecAttn (decode_state.h) only HD is read ahead of that."""
