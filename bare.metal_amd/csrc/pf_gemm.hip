@@ -184,13 +184,16 @@ __global__ __launch_bounds__(PNTH, pfg_waves(QF, EPI, MI, NJ)) void k_pf_gemm(Pf
     };
     /* The first three steps' operands are on their way before anything that
      * only the epilogue reads: loads return in order, and the K loop's first
-     * wait must not be for those. */
+     * wait must not be for those.  A wave with fewer steps asks for no more:
+     * nothing hides those loads (the o projection at 135M, nine steps for
+     * four waves, 512 tokens: 4.84 us without them before this order, 5.56
+     * with, 4.9-5.1 now; q/k/v 6.1 -> 5.9). */
     PfgStage<QF, MI, NJ> s0, s1, s2;
     load(s_beg, s0);
     __builtin_amdgcn_sched_barrier(0);
     load(s_beg + 1, s1);
     __builtin_amdgcn_sched_barrier(0);
-    load(s_beg + 2, s2);
+    if (s_end - s_beg > 2) load(s_beg + 2, s2);
     __builtin_amdgcn_sched_barrier(0);
     /* Epilogue thread map: row r of the tile; CPT columns from c0 (8 gate
      * and 8 up columns from j0 for SwiGLU). */
@@ -203,13 +206,14 @@ __global__ __launch_bounds__(PNTH, pfg_waves(QF, EPI, MI, NJ)) void k_pf_gemm(Pf
     const bool whole = (EPI == PFG_STORE || EPI == PFG_RESID || (EPI == PFG_QKV && p == 0)) && n0 + c0 + CPT <= N &&
                        ((uintptr_t)dst & 15) == 0;
     /* What the epilogue reads, loaded ahead of the K loop.  A launch with a
-     * residual: its rows and, when it writes the next norm's operand, that
-     * norm's weights; a thread's CPT columns lie inside N or past it (N is a
-     * multiple of 32), and past it the last ones are read for nothing. */
+     * residual: its rows (threads past the tile's read its last one) and, when
+     * it writes the next norm's operand, that norm's weights; a thread's CPT
+     * columns lie inside N or past it (N is a multiple of 32), and past it the
+     * last ones are read for nothing. */
     f32x4 res[CPT / 4], gnr[CPT / 4];
     if (EPI == PFG_RESID) {
         const int cc = max(min(n0 + c0, N - CPT), 0);
-        const float* rp = a.x + (size_t)min(m, M - 1) * ldc + cc;
+        const float* rp = a.x + (size_t)min(m0 + min(r, PTM - 1), M - 1) * ldc + cc;
         const float* gp = a.an ? a.gn + cc : rp; /* no branch around a load: the waits would be for the worse case */
 #pragma unroll
         for (int c = 0; c < CPT / 4; c++) res[c] = __builtin_bit_cast(f32x4, ld16<4>(rp + 4 * c));
