@@ -145,7 +145,7 @@ __global__ __launch_bounds__(NT) void k_rmsnorm(const float* __restrict__ x, con
 typedef float ew_f32x4 __attribute__((ext_vector_type(4)));
 
 /* The same where rows and weights are whole 16-byte groups (C a multiple of
- * 4, at most 4 * NT * NV): a row is read once, NV groups per thread kept in
+ * 4 past 64, at most 4 * NT * NV): a row is read once, NV groups per thread kept in
  * registers with the weights, which do not wait for the sum.  What bounds it
  * is that chain of loads: 1 row of 576 2.6 -> 1.8 us, 333 rows of 960 4.3 -> 3.0 us
  * (kernel trace).  Add and SwiGLU four elements a thread measured no faster
@@ -1666,7 +1666,8 @@ extern "C" int bmk_launch_rmsnorm(const bmk_launch_t* a) {
     BMK_NEED_BYTES(a, 2, (size_t)N * C * 4, "out");
     const ew_f32x4 *x4 = (const ew_f32x4*)a->dev[0], *w4 = (const ew_f32x4*)a->dev[1];
     ew_f32x4* o4 = (ew_f32x4*)a->dev[2];
-    const bool vec = C % 4 == 0 && (((uintptr_t)x4 | (uintptr_t)w4 | (uintptr_t)o4) & 15) == 0;
+    /* rows of up to 64 columns fill no more lanes in groups: 2048 x 32 2.88 us, 3.02 in groups */
+    const bool vec = C > 64 && C % 4 == 0 && (((uintptr_t)x4 | (uintptr_t)w4 | (uintptr_t)o4) & 15) == 0;
     if (vec && C <= 4 * NT)
         hipLaunchKernelGGL(k_rmsnorm4<1>, dim3(N), dim3(NT), 0, a->stream, x4, w4, o4, C / 4, eps);
     else if (vec && C <= 16 * NT)
