@@ -657,9 +657,11 @@ extern "C" int mv_tiles_for(int OC, int C, int U) {
  * against 9.8 (x576); 1 or 2 rows per lane are slower, 16 too.
  * At the other end a launch is one workgroup's chain, and rows in flight
  * only lengthen it: one row per lane where that fills at most one workgroup
- * per CU, else two.  Back to back, 4 rows / now (us): 576 x 576 4.07 / 3.45, 1536 x
- * 576 4.08 / 3.41, 576 x 1536 4.35 / 3.51, 960 x 960 4.22 / 3.52, 2560 x 960 (two rows) 4.21
- * / 3.85, 960 x 2560 4.45 / 3.89; one row there, 320 workgroups, 4.46. */
+ * per CU, else two.  Kernel trace, weights in cache / not, 4 rows -> now (us): 576 x
+ * 576 4.1 / 4.3 -> 3.5 / 3.5, 1536 x 576 4.2 / 4.5 -> 3.6 / 3.6, 576 x 1536 4.6 / 4.8 -> 3.7 / 3.7,
+ * 960 x 960 4.4 / 4.8 -> 3.8 / 3.9, 2560 x 960 (two rows) 4.2 / 4.8 -> 4.1 / 4.2, 960 x 2560 4.7 /
+ * 4.9 -> 4.0 / 4.1.  Calls that the host issues one by one come no faster than it
+ * issues them, 4.1 us apart here, 4.9 in another program: those do not show it. */
 #define MV_WIDE_MIN_TILES 768
 #define MV_CUS 256
 
