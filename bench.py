@@ -185,7 +185,7 @@ def _timed_loop(fn, budget: float):
 def cpu_baseline(wls, seconds: float, threads: int):
     """The main line's whole token on the host: the oracle's fp32 SIMD +
     OpenMP restatement of the same Q8 arithmetic, at 1 thread and at
-    `threads` (the GPU box's CPU share), over a time-bounded sample.  The
+    `threads` (this process's CPU share), over a time-bounded sample.  The
     weight copies are used in turn, as on the GPU: one 407 MB copy split over
     16 threads is about 25 MB per thread, which a chiplet's L3 keeps from one
     pass to the next, so repeating one copy would time the caches."""

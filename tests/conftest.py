@@ -11,7 +11,7 @@ for p in (ROOT, os.path.join(ROOT, "oracle")):  # bmhip (the ctypes wrapper) and
 
 
 def pytest_configure(config):
-    config.addinivalue_line("markers", "gpu: needs an MI355X (run on the GPU box)")
+    config.addinivalue_line("markers", "gpu: needs an MI355X")
 
 
 @pytest.fixture(scope="session")
